@@ -47,6 +47,7 @@ MFMA_VGPR = ["-mllvm", "-amdgpu-mfma-vgpr-form"]
 SOURCES = (
     ("g1env.hip", ILP_FIRST),
     ("rollout_kernel.hip", ILP_FIRST + MFMA_VGPR),
+    ("resident_kernel.hip", ILP_FIRST),
 )
 
 

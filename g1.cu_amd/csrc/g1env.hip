@@ -37,6 +37,7 @@ static void fail(const char* msg) {
 }
 
 #include "queue.h"
+#include "resident.h"
 
 constexpr int kStepChunks = 4;     // host-step copies between pageable and pinned memory, pipelined
 
@@ -153,9 +154,10 @@ __global__ void k_pack_tiles(TilePackArgs a) {
 }
 
 // Pack torch-order weights (W0, b0, .., Wmu, bmu, Wv, bv, log_std) of a policy of nl hidden layers
-// into the wide tile's layout (WideLayout).
+// into the wide tile's layout (WideLayout). chain: each 16-row, 16-input block transposed for k_resident,
+// whose lanes read one k-step of the four lane groups at once: [e][row][g] instead of [g][row][e].
 struct WidePackArgs {
-  const float* W; const float* mean; const float* var; float* Wt; WideLayout wl; int hid[kMaxLayers];
+  const float* W; const float* mean; const float* var; float* Wt; WideLayout wl; int hid[kMaxLayers]; int chain;
 };
 __global__ void k_pack_wide(WidePackArgs a) {
   const long idx = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -194,10 +196,11 @@ __global__ void k_pack_wide(WidePackArgs a) {
         else v = row < kAct ? a.W[oW + (long)kAct * in + row] : (row == kAct ? a.W[oWv + in] : 0.f);
       } else {
         const long rel = idx - T.woff[Ly];
-        const int e = (int)(rel & 3), lane = (int)((rel >> 2) & 63);
+        const int lo = (int)(rel & 3), hi = (int)((rel >> 6) & 3);
+        const int e = a.chain ? hi : lo, g = a.chain ? lo : hi;
         const long rq = rel >> 8;
         const int qd = (int)(rq % T.nQ[Ly]), ot = (int)(rq / T.nQ[Ly]);
-        const int row = 16 * ot + (lane & 15), k = tile_kappa(Ly, 4 * qd + e, lane >> 4);
+        const int row = 16 * ot + (int)((rel >> 2) & 15), k = tile_kappa(Ly, 4 * qd + e, g);
         if (k < in) {
           if (!head) v = row < a.hid[Ly] ? a.W[oW + (long)row * in + k] : 0.f;
           else v = row < kAct ? a.W[oW + (long)row * in + k] : (row == kAct ? a.W[oWv + k] : 0.f);
@@ -567,7 +570,8 @@ struct EnvState {
   float *qacc_e, *qacc_vx;
   unsigned qdone;   // value of every pair flag after the launches enqueued so far
   int qpar;         // counter row of the next launch
-  int pgrid;        // persistent grid: resident blocks of k_physics, a multiple of kQueues
+  int waves;        // blocks of k_physics resident on the chip, a multiple of kQueues
+  int pgrid;        // persistent grid: those blocks, no more than the pairs need
   int xlocal;       // blocks land on XCD blockIdx % kXcds (measured at creation)
   int fences;       // 1: hand over state with agent-scope fences even where xlocal holds
   // one-launch rollout (k_rollout): policy tiles' flags, their completed-step count, packed weights
@@ -797,9 +801,9 @@ static void poll_queue_error(EnvState* E) {
 // The one-launch rollout runs policies of two hidden layers of at most 256 units each on the
 // register-resident tile (policy_tile, at 256-256 with zero padding) and every other accepted shape
 // (1..3 hidden layers of at most 512 units) on the wide tile (policy_tile_wide, activations staged
-// in global memory). The split form (policy and physics launches per control step) remains for
-// g1_env_set_fused(h, 0) and for g1_rollout_noalloc with a wide shape (the wide tile's activation
-// buffers are allocated by the library).
+// in global memory); small batches of either kind run resident waves (resident_worlds). The split form
+// (policy and physics launches per control step) remains for g1_env_set_fused(h, 0) and for
+// g1_rollout_noalloc with a wide shape (the wide tile's activation buffers are allocated by the library).
 static bool narrow_shape(const PolicyShape& sh) {
   return sh.nl == 2 && sh.hid[0] <= kTileMaxHidden && sh.hid[1] <= kTileMaxHidden;
 }
@@ -813,6 +817,59 @@ static int tiles_per_queue(int N) {
   return (nq + kTilePairs - 1) / kTilePairs;
 }
 
+// Room for `total` floats of packed policy weights: wp (capacity wp_cap) or, with wp null, the env's own
+// buffer, grown with hipMalloc.
+static float* packed_buffer(EnvState* E, long total, float* wp, long wp_cap) {
+  if (wp) {
+    if (total > wp_cap) fail("rollout: packed policy larger than its buffer");
+    return wp;
+  }
+  if (total > E->Wt_cap) {
+    if (E->Wt) dev_free(E, E->Wt, E->Wt_cap * sizeof(float));
+    dev_alloc(E, &E->Wt, total * sizeof(float));
+    E->Wt_cap = total;
+  }
+  return E->Wt;
+}
+
+static void pack_wide(EnvState* E, const float* W, const float* mean, const float* var, float* Wt,
+                      const WideLayout& wl, bool chain) {
+  WidePackArgs pk{W, mean, var, Wt, wl, {0, 0, 0, 0}, chain ? 1 : 0};
+  for (int i = 0; i < E->shape.nl; ++i) pk.hid[i] = E->shape.hid[i];
+  hipLaunchKernelGGL(k_pack_wide, dim3((unsigned)((wl.total + 255) / 256)), dim3(256), 0, 0, pk);
+  HIPCHECK(hipGetLastError());
+}
+
+// Worlds per wave of the resident form (k_resident), or 0 where the work queue runs the rollout: one while
+// every wave can have a SIMD to itself (1024 worlds), two while all waves are resident at once (4096).
+// Measured, ms per 32 steps of the 256-256 policy with one world per wave, two, and the queue: 1024
+// worlds 3.38, 3.85, 5.42; 1536 3.86, 3.87, 5.48; 2048 3.99, 3.81, 5.51; 4096 -, 4.46, 6.02; past that
+// a second round of waves would start when the first ends, and the queue spreads the work evenly (8192
+// worlds 7.6). An env set to the fenced hand-over keeps the queue, which that mode is about.
+static int resident_worlds(const EnvState* E) {
+  if (E->fences) return 0;
+  return E->N <= E->waves / 2 ? 1 : (E->N <= 2 * E->waves ? 2 : 0);
+}
+
+// The whole rollout as one k_resident launch on the null stream; wp as in rollout_fused.
+static void rollout_resident(EnvState* E, int per_wave, int H, const float* W, const float* mean, const float* var,
+                             float* O, float* A, float* LP, float* V, float* R, float* D, float* Vlast,
+                             const float* act_noise, const float* reset_noise, float* wp, long wp_cap) {
+  const WideLayout wl = wide_layout(E->shape.nl, E->shape.hid, E->shape.act);
+  float* Wt = packed_buffer(E, wl.total, wp, wp_cap);
+  pack_wide(E, W, mean, var, Wt, wl, true);
+  ResidentArgs ra{};
+  ra.ph = phys_args(E);
+  PhysArgs& a = ra.ph;
+  a.K = H; a.t0 = 0; a.astep = 1; a.rstep = 1; a.R = R; a.D = D; a.reset_noise = reset_noise;
+  ra.po = TileArgs{Wt, TileLayout{}, act_noise, O, A, LP, V, Vlast, H, 1, wl, nullptr};
+  const bool prof = E->prof_on != 0 && !wp;
+  if (prof) prof_mark(E->ev_phys, E->n_phys);
+  launch_resident_kernel(ra, per_wave == 2);
+  HIPCHECK(hipGetLastError());
+  if (prof) prof_mark(E->ev_phys, E->n_phys);
+}
+
 // The whole rollout as one k_rollout launch on the null stream; wp (capacity wp_cap floats) takes
 // the tile-packed weights instead of the env's own buffer.
 static void rollout_fused(EnvState* E, int H, const float* W, const float* mean, const float* var, float* O, float* A,
@@ -822,17 +879,7 @@ static void rollout_fused(EnvState* E, int H, const float* W, const float* mean,
   const TileLayout tl = tile_layout(E->shape.act);
   const WideLayout wl = wide_layout(E->shape.nl, E->shape.hid, E->shape.act);
   const long total = wide ? wl.total : tl.total;
-  float* Wt = wp;
-  if (!Wt) {
-    if (total > E->Wt_cap) {
-      if (E->Wt) dev_free(E, E->Wt, E->Wt_cap * sizeof(float));
-      dev_alloc(E, &E->Wt, total * sizeof(float));
-      E->Wt_cap = total;
-    }
-    Wt = E->Wt;
-  } else if (total > wp_cap) {
-    fail("rollout: tile-packed policy larger than its buffer");
-  }
+  float* Wt = packed_buffer(E, total, wp, wp_cap);
   float* scr = nullptr;
   if (wide) {
     if (wp) fail("rollout: the wide one-launch policy needs the library's activation buffers");
@@ -843,14 +890,12 @@ static void rollout_fused(EnvState* E, int H, const float* W, const float* mean,
       E->scr_cap = need;
     }
     scr = E->scr;
-    WidePackArgs pk{W, mean, var, Wt, wl, {0, 0, 0, 0}};
-    for (int i = 0; i < E->shape.nl; ++i) pk.hid[i] = E->shape.hid[i];
-    hipLaunchKernelGGL(k_pack_wide, dim3((unsigned)((wl.total + 255) / 256)), dim3(256), 0, 0, pk);
+    pack_wide(E, W, mean, var, Wt, wl, false);
   } else {
     TilePackArgs pk{W, mean, var, Wt, tl, E->shape.hid[0], E->shape.hid[1]};
     hipLaunchKernelGGL(k_pack_tiles, dim3((unsigned)((tl.total + 255) / 256)), dim3(256), 0, 0, pk);
+    HIPCHECK(hipGetLastError());
   }
-  HIPCHECK(hipGetLastError());
   RolloutArgs ra{};
   ra.ph = phys_args(E);
   PhysArgs& a = ra.ph;
@@ -882,6 +927,10 @@ static void rollout_impl(EnvState* E, int H, const float* W, const float* mean, 
   poll_queue_error(E);
   if (H < 0) H = 0;   // no control step; the bootstrap value is still computed (as the reference's k_rollout)
   if (E->fused && fused_shape(E->shape, wp != nullptr)) {
+    if (const int per_wave = resident_worlds(E)) {
+      rollout_resident(E, per_wave, H, W, mean, var, O, A, LP, V, R, D, Vlast, act_noise, reset_noise, wp, wp_cap);
+      return;
+    }
     rollout_fused(E, H, W, mean, var, O, A, LP, V, R, D, Vlast, act_noise, reset_noise, wp, wp_cap);
     return;
   }
@@ -974,6 +1023,7 @@ void* g1_env_create(int N, int substeps, int pgs_iters, unsigned long seed) {
     int cap = (cus * (per_cu > 0 ? per_cu : 1)) / kQueues * kQueues;
     if (cap < kQueues) cap = kQueues;
     const int need = (npairs + kQueues - 1) / kQueues * kQueues;
+    E->waves = cap;
     E->pgrid = need < cap ? need : cap;
     // placement of the blocks on the XCDs: round-robin lets each queue hand over state in one L2
     int* dx = nullptr;
@@ -1146,6 +1196,8 @@ void g1_occupancy_report(void) {
   struct { const char* nm; const void* fn; int threads; size_t smem; } ks[] = {
       {"k_rollout", rollout_kernel_fn(false), kPhysThreads, 0},
       {"k_rollout (wide)", rollout_kernel_fn(true), kPhysThreads, 0},
+      {"k_resident (1)", resident_kernel_fn(false), kPhysThreads, 0},
+      {"k_resident (2)", resident_kernel_fn(true), kPhysThreads, 0},
       {"k_physics", (const void*)k_physics, kPhysThreads, 0},
       {"k_policy", (const void*)k_policy, kPolicyThreads, policy_smem(PolicyShape{2, {256, 256, 0, 0}, 0})},
       {"k_probe", (const void*)k_probe, kPhysThreads, 0}};

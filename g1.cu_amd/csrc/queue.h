@@ -92,12 +92,79 @@ __device__ __forceinline__ void release_flag(unsigned* flag, unsigned value, int
   if (threadIdx.x == 0) __hip_atomic_store(flag, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// PD target of the lane's hinge = clamp(stand + 0.5 a) (reference: src/g1_env.cu:123-130)
+__device__ __forceinline__ float pd_target(const LaneModel& L, float act) {
+  float target = fmaf_(0.5f, act, L.qstand);
+  if (target < L.clo) target = L.clo;
+  if (target > L.chi) target = L.chi;
+  return target;
+}
+
+// Substeps [s0, s1) of a control step of the lane's world: PD torques, world_qacc, Euler (reference:
+// src/g1_env.cu:141-163). Adds to the step's energy and base-velocity sums; returns the contacts at
+// the last substep. hcnt: lane q < 9 counts the world's substeps with q contacts.
+__device__ __forceinline__ int run_substeps(const SolveParams& P, WorldLds& s, const LaneModel& L, int l, bool wvalid,
+                                            float target, int s0, int s1, LaneState& st, float& energy, float& vx_sum,
+                                            unsigned& hcnt) {
+  int nc_last = 0;
+#pragma unroll 1
+  for (int sub = s0; sub < s1; ++sub) {
+    float jtau = 0.f;
+    if (L.hinge) {
+      float pdt = fmaf_(-L.kd, st.jqd, L.kp * (target - st.jq));
+      if (pdt < L.flo) pdt = L.flo;
+      else if (pdt > L.fhi) pdt = L.fhi;
+      jtau = pdt;
+      energy += fabsf(pdt * st.jqd);
+    }
+    float bqacc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, jqacc = 0.f;
+    const int nc = world_qacc(l, s, st, jtau, P, bqacc, jqacc);
+    hcnt += (l == nc && wvalid) ? 1u : 0u;
+    nc_last = nc;
+    integrate_lane(L, st, bqacc, jqacc, true);
+    vx_sum += st.bqd[0];
+  }
+  return nc_last;
+}
+
+// The observation of the world's state, each lane writing its own entries (the values of k_obs).
+__device__ __forceinline__ void store_observation(float* o, const LaneModel& L, int l, const LaneState& st, float pa) {
+  if (l == 1) {
+#pragma unroll
+    for (int m = 0; m < 6; ++m) o[m] = st.bqd[m];
+    const float qw = st.bq[3], qx = st.bq[4], qy = st.bq[5], qz = st.bq[6];
+    o[6] = -(2.f * fmaf_(-qw, qy, qx * qz));
+    o[7] = -(2.f * fmaf_(qw, qx, qy * qz));
+    o[8] = -fmaf_(-2.f, fmaf_(qy, qy, qx * qx), 1.f);
+  }
+  if (L.hinge) {
+    const int ai = L.b - 2;
+    o[9 + ai] = st.jq; o[38 + ai] = st.jqd; o[67 + ai] = pa;
+  }
+  if (l == 0) { o[96] = 0.8f; o[97] = 0.f; o[98] = 0.f; o[99] = 0.f; }
+}
+
+// The world's state back to its rows: lane 1 the free joint, each hinge lane its joint.
+__device__ __forceinline__ void store_state(const PhysArgs& a, const LaneModel& L, int l, int w, const LaneState& st) {
+  float* oq = a.qp + (long)w * kNQ;
+  float* ov = a.qv + (long)w * kNV;
+  if (l == 1) {
+#pragma unroll
+    for (int m = 0; m < 7; ++m) oq[m] = st.bq[m];
+#pragma unroll
+    for (int m = 0; m < 6; ++m) ov[m] = st.bqd[m];
+  }
+  if (L.hinge) {
+    oq[L.b + 5] = st.jq;
+    ov[L.b + 4] = st.jqd;
+  }
+}
+
 // One physics work item: world pair p (the two 32-lane groups of the wave), control step k of the
-// launch, substeps [cst[c], cst[c + 1]) of it: PD torques, world_qacc, Euler; the last chunk of a
-// control step adds the step's reward, termination and auto-reset (reference:
-// src/g1_env.cu:118-212, the k_rollout substep loop :319-325). Every input a previous item or launch
-// wrote is read from the L2 (the actions too: in k_rollout the policy items of the same launch
-// write them).
+// launch, substeps [cst[c], cst[c + 1]) of it; the last chunk of a control step adds the step's
+// reward, termination and auto-reset (reference: src/g1_env.cu:118-212, the k_rollout substep loop
+// :319-325). Every input a previous item or launch wrote is read from the L2 (the actions too: in
+// k_rollout the policy items of the same launch write them).
 __device__ __forceinline__ void physics_item(const PhysArgs& a, WorldLds& s, const LaneModel& L, int g, int l, int w,
                                              int k, int c, unsigned& hcnt) {
   const int ai = L.hinge ? L.b - 2 : 0;
@@ -116,10 +183,7 @@ __device__ __forceinline__ void physics_item(const PhysArgs& a, WorldLds& s, con
   st.jqd = L.hinge ? ld_l2(gv + L.b + 4) : 0.f;
   const int t = a.t0 + k * a.astep;
   const float act = L.hinge ? ld_l2(a.act + ((long)t * a.N + wc) * kAct + ai) : 0.f;
-  // PD target = clamp(stand + 0.5 a) (reference: src/g1_env.cu:123-130)
-  float target = fmaf_(0.5f, act, L.qstand);
-  if (target < L.clo) target = L.clo;
-  if (target > L.chi) target = L.chi;
+  const float target = pd_target(L, act);
   float vx_sum = 0.f, energy = 0.f;
   if (c > 0) {
     energy = ld_l2(a.acc + (long)wc * kGroup + l);
@@ -128,34 +192,19 @@ __device__ __forceinline__ void physics_item(const PhysArgs& a, WorldLds& s, con
   const bool lastk = k == a.K - 1;   // the launch's last control step has a chunk table of its own
   const int nck = lastk ? a.nchl : a.nch;
   const int s0 = lastk ? a.cstl[c] : a.cst[c], s1 = lastk ? a.cstl[c + 1] : a.cst[c + 1];
-  int nc_last = 0;   // the world's contacts at its last substep
-#pragma unroll 1
-  for (int sub = s0; sub < s1; ++sub) {
-    float jtau = 0.f;
-    if (L.hinge) {
-      float pdt = fmaf_(-L.kd, st.jqd, L.kp * (target - st.jq));
-      if (pdt < L.flo) pdt = L.flo;
-      else if (pdt > L.fhi) pdt = L.fhi;
-      jtau = pdt;
-      energy += fabsf(pdt * st.jqd);
-    }
-    float bqacc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, jqacc = 0.f;
-    const int nc = world_qacc(l, s, st, jtau, P, bqacc, jqacc);
-    hcnt += (l == nc && wvalid) ? 1u : 0u;
-    nc_last = nc;
-    integrate_lane(L, st, bqacc, jqacc, true);
-    vx_sum += st.bqd[0];
-  }
+  const int nc_last = run_substeps(P, s, L, l, wvalid, target, s0, s1, st, energy, vx_sum, hcnt);
   if (c < nck - 1) {
     if (wvalid) {
       a.acc[(long)w * kGroup + l] = energy;
       if (l == 1) a.vxs[w] = vx_sum;
     }
   } else {
-    // ---- reward / termination / auto-reset (reference: src/g1_env.cu:164-211), lane 1 decides
     float pa = L.hinge ? ld_l2(a.pa + (long)wc * kAct + ai) : 0.f;
     int step = ld_l2(a.steps + wc);
     unsigned rng = ld_l2(a.rng + wc);
+    // ---- reward / termination / auto-reset (reference: src/g1_env.cu:164-211), lane 1 decides. The
+    // statements of finish_control_step (resident.h), written out: called here they compile to another
+    // schedule of the item, 0.4% slower (config 3 7.61 -> 7.65 ms).
     const float da = L.hinge ? act - pa : 0.f;
     float act_pen = gsum(da * da);
     const float energy_tot = gsum(energy);
@@ -205,36 +254,10 @@ __device__ __forceinline__ void physics_item(const PhysArgs& a, WorldLds& s, con
         a.rng[w] = rng;
       }
       if (L.hinge) a.pa[(long)w * kAct + ai] = pa;
-      if (a.obs && k == a.K - 1) {
-        // observation of the final state, each lane writing its own entries (same values as k_obs)
-        float* o = a.obs + (long)w * kObs;
-        if (l == 1) {
-#pragma unroll
-          for (int m = 0; m < 6; ++m) o[m] = st.bqd[m];
-          const float qw = st.bq[3], qx = st.bq[4], qy = st.bq[5], qz = st.bq[6];
-          o[6] = -(2.f * fmaf_(-qw, qy, qx * qz));
-          o[7] = -(2.f * fmaf_(qw, qx, qy * qz));
-          o[8] = -fmaf_(-2.f, fmaf_(qy, qy, qx * qx), 1.f);
-        }
-        if (L.hinge) { o[9 + ai] = st.jq; o[38 + ai] = st.jqd; o[67 + ai] = pa; }
-        if (l == 0) { o[96] = 0.8f; o[97] = 0.f; o[98] = 0.f; o[99] = 0.f; }
-      }
+      if (a.obs && k == a.K - 1) store_observation(a.obs + (long)w * kObs, L, l, st, pa);
     }
   }
-  if (wvalid) {
-    float* oq = a.qp + (long)w * kNQ;
-    float* ov = a.qv + (long)w * kNV;
-    if (l == 1) {
-#pragma unroll
-      for (int m = 0; m < 7; ++m) oq[m] = st.bq[m];
-#pragma unroll
-      for (int m = 0; m < 6; ++m) ov[m] = st.bqd[m];
-    }
-    if (L.hinge) {
-      oq[L.b + 5] = st.jq;
-      ov[L.b + 4] = st.jqd;
-    }
-  }
+  if (wvalid) store_state(a, L, l, w, st);
 }
 
 // ====================================================================== the rollout in one launch

@@ -1,0 +1,84 @@
+// resident_kernel.hip -- k_resident, a whole rollout with one or two worlds per wave (resident.h). Its own
+// translation unit for the wavefront-fence phase boundaries.
+#include <hip/hip_runtime.h>
+
+#define G1_PHASE_FENCE   // world_qacc's phase boundaries as wavefront fences (see wave_sync)
+#include "resident.h"
+
+namespace g1k {
+
+// kW: worlds per wave. With two, group g of block b has world 2 b + g; with one, both groups carry world
+// b and group 0 stores: the second group costs nothing (its lanes would idle), and the wave then runs
+// the contact phases at its own world's contact count instead of the larger of two.
+template <int kW>
+__global__ void __launch_bounds__(kPhysThreads) k_resident(ResidentArgs ra) {
+  __shared__ __align__(16) WorldLds lds[2];
+  const int g = group_id(), l = group_lane();
+  WorldLds& s = lds[g];
+  const int N = ra.ph.N;
+  const int w = kW == 2 ? 2 * (int)blockIdx.x + g : (int)blockIdx.x;
+  const bool wvalid = kW == 2 ? w < N : g == 0;
+  const int wc = w < N ? w : N - 1;   // an odd N's last group repeats world N - 1 and stores nothing
+  const bool hinge = l >= 2 && l < kNBody;
+  LaneState st;
+  float pa;
+  int step;
+  unsigned rng;
+  {
+    const PhysArgs& a = ra.ph;
+    const float* gq = a.qp + (long)wc * kNQ;
+    const float* gv = a.qv + (long)wc * kNV;
+#pragma unroll
+    for (int m = 0; m < 7; ++m) st.bq[m] = gq[m];
+#pragma unroll
+    for (int m = 0; m < 6; ++m) st.bqd[m] = gv[m];
+    st.jq = hinge ? gq[l + 5] : 0.f;
+    st.jqd = hinge ? gv[l + 4] : 0.f;
+    pa = hinge ? a.pa[(long)wc * kAct + l - 2] : 0.f;
+    step = a.steps[wc];
+    rng = a.rng[wc];
+  }
+  unsigned hcnt = 0;
+  const int K = ra.ph.K;
+#pragma unroll 1
+  for (int k = 0;; ++k) {
+    const ResidentArgs& rb = kernarg_reread<ResidentArgs>();
+    const float act =
+        wave_policy<kW>(rb.po, st, pa, rng, rb.ph.seed, rb.ph.N, k, w, wc, wvalid, reinterpret_cast<float*>(lds));
+    if (k >= K) break;   // the bootstrap value of the state after the last step
+    // the lane's model constants, formed here (opaque lane index) rather than held across steps
+    int lo = l;
+    __asm__ volatile("" : "+v"(lo));
+    const LaneModel L = lane_model(lo);
+    const PhysArgs& a = kernarg_reread<ResidentArgs>().ph;
+    float vx_sum = 0.f, energy = 0.f;
+    const SolveParams P{a.pgs, a.mu, true, true};
+    run_substeps(P, s, L, l, wvalid, pd_target(L, act), 0, a.S, st, energy, vx_sum, hcnt);
+    float r;
+    const int done = finish_control_step(a, L, l, wc, k, act, vx_sum, energy, st, pa, step, rng, r);
+    if (wvalid && l == 1) {
+      a.R[(long)k * a.N + w] = r;
+      a.D[(long)k * a.N + w] = (float)done;
+    }
+  }
+  const PhysArgs& a = kernarg_reread<ResidentArgs>().ph;
+  if (wvalid && a.K > 0) {
+    const LaneModel L = lane_model(l);
+    store_state(a, L, l, w, st);
+    if (L.hinge) a.pa[(long)w * kAct + l - 2] = pa;
+    if (l == 1) {
+      a.steps[w] = step;
+      a.rng[w] = rng;
+    }
+  }
+  if (a.ncon_hist && l < 9 && hcnt) atomicAdd(&a.ncon_hist[l], (unsigned long long)hcnt);
+}
+
+void launch_resident_kernel(const ResidentArgs& ra, bool two) {
+  if (two) hipLaunchKernelGGL(k_resident<2>, dim3((unsigned)(ra.ph.N + 1) / 2), dim3(kPhysThreads), 0, 0, ra);
+  else hipLaunchKernelGGL(k_resident<1>, dim3((unsigned)ra.ph.N), dim3(kPhysThreads), 0, 0, ra);
+}
+
+const void* resident_kernel_fn(bool two) { return two ? (const void*)k_resident<2> : (const void*)k_resident<1>; }
+
+}  // namespace g1k

@@ -117,12 +117,14 @@ int g1_env_check(void* h);
 /* State hand-over between the physics work items: fences = 0 hands a world pair's state over in
  * the L2 of its queue's XCD (the default; needs the round-robin block placement verified at
  * creation), fences = 1 uses agent-scope release/acquire fences (correct on any placement,
- * slower). Returns 0, or -1 when the mode is unavailable. */
+ * slower) and keeps the queue also for small batches, whose rollouts hand nothing over otherwise (see
+ * g1_env_set_fused). Results are the same bit for bit. Returns 0, or -1 when the mode is unavailable. */
 int g1_env_set_handover(void* h, int fences);
 
 /* Rollout form: on = 1 (the default) runs g1_rollout as one persistent launch that interleaves the
- * policy of 16-world tiles with the physics work items; on = 0 launches the policy and the physics
- * once per control step. The one-launch form covers every shape g1_env_set_policy accepts (two
+ * policy of 16-world tiles with the physics work items, or, for batches that fit the chip at one or two
+ * worlds per wave (up to 4096), keeps each wave's worlds for the whole launch (the same results bit for
+ * bit); on = 0 launches the policy and the physics once per control step. The one-launch form covers every shape g1_env_set_policy accepts (two
  * hidden layers of at most 256 units on a register-resident tile, other shapes on a tile that
  * stages its activations in library-allocated device memory); g1_rollout_noalloc runs the latter
  * shapes in the per-step form. Returns 0, 1 when on = 1 but the current policy shape takes the

@@ -1,0 +1,62 @@
+"""Rollouts of batches that fit the chip at one or two worlds per wave (k_resident, up to 4096 worlds) against
+the work-queue form (k_rollout), which the fenced hand-over keeps at every size: every trajectory output, the
+final state and the contact histogram bit for bit. The two forms share the physics, and the policy's sums run
+in the same order on the vector ALUs as on v_mfma_f32_16x16x4f32, so the tolerance is zero."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def g1():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import g1env
+    return g1env
+
+
+def _dev(x):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(x)).cuda()
+
+
+# the smallest batches; both sides of one world per wave and of two (odd counts leave half a wave); layers
+# of one to eight row blocks, ragged widths, one to three hidden layers; a horizon of zero
+@pytest.mark.parametrize("N,H,S,hidden,act,given", [
+    (1, 3, 10, (256, 256), 0, False), (3, 2, 4, (17, 1), 1, True), (1023, 2, 5, (200, 72), 1, False),
+    (1024, 2, 5, (256, 256), 0, True), (1025, 2, 5, (512, 512, 256), 1, True), (2047, 2, 4, (300,), 0, False),
+    (4095, 2, 4, (64, 513 - 1, 130), 0, False), (4096, 3, 3, (256, 256), 0, False), (40, 0, 10, (128, 65), 1, False),
+    (130, 12, 10, (256, 256), 0, False)])
+def test_resident_rollout_equals_work_queue(g1, N, H, S, hidden, act, given):
+    import configs
+    import torch
+    rng = np.random.default_rng(N + H)
+    qp, qv, pa, steps = configs.reset_states(rng, N)
+    qv = rng.normal(0, 0.3, qv.shape).astype(np.float32)
+    pa = rng.normal(0, 0.3, pa.shape).astype(np.float32)
+    steps[::5] = 998        # time-outs and auto-resets inside the horizon
+    W = _dev(configs.policy_init(rng, hidden=hidden))
+    mean, var = _dev(rng.normal(0, 0.1, 100).astype(np.float32)), _dev(rng.uniform(0.5, 2.0, 100).astype(np.float32))
+    an, rn = (_dev(x) for x in configs.rollout_noise(rng, H, N)) if given else (None, None)
+    got = []
+    for fences in (0, 1):
+        with g1.Env(N, substeps=S, pgs_iters=8, seed=9) as env:
+            env.set_policy(hidden, act)
+            env.set_handover(fences)
+            env.set_state(qp, qv, pa, steps)
+            env.ncon_hist(enable=True)
+            out = []
+            for _ in range(2):   # the second continues from the first's state and noise counters
+                tr = g1.Trajectory(H, N)
+                for t in tr.tensors():
+                    t.fill_(7.0)
+                tr.run(env, W, mean, var, an, rn)
+                torch.cuda.synchronize()
+                out += [tr.numpy()[f].view(np.uint32) for f in tr.FIELDS]
+            got.append(out + [x.view(np.uint32) for x in env.get_state()] + [env.ncon_hist(enable=False)])
+            assert env.check() == 0
+    for i, (a, b) in enumerate(zip(*got)):
+        assert np.array_equal(a, b), i
+    assert H == 0 or (got[0][5] != 0).any()   # some world finished
