@@ -761,10 +761,29 @@ static void chunk_schedule(PhysArgs& a, int pgrid, bool one_launch = false) {
   a.nchl = build(big ? 1 : 2, a.cstl);
 }
 
+// Worlds per wave of the resident form (k_resident), or 0 where the work queue runs the launch: one while
+// every wave can have a SIMD to itself (1024 worlds), two while all waves are resident at once (4096).
+// Measured, ms per 32 steps of the 256-256 policy with one world per wave, two, and the queue: 1024
+// worlds 3.38, 3.85, 5.42; 1536 3.86, 3.87, 5.48; 2048 3.99, 3.81, 5.51; 4096 -, 4.46, 6.02; past that
+// a second round of waves would start when the first ends, and the queue spreads the work evenly (8192
+// worlds 7.6). Control steps on given actions, us per 20 steps of standing robots: 64 worlds 3452, 3504,
+// 3599; 1024 3615, 3696, 3758; 2048 4162, 3604, 3723; 4096 -, 4176, 4224. An env set to the fenced hand-over keeps the queue, which that mode is about.
+static int resident_worlds(const EnvState* E) {
+  if (E->fences) return 0;
+  return E->N <= E->waves / 2 ? 1 : (E->N <= 2 * E->waves ? 2 : 0);
+}
+
 // Enqueue one physics launch on the null stream; the queue state (flag base, counter row) advances
 // on the host in launch order, which is the stream's execution order.
 static void launch_physics(EnvState* E, PhysArgs& a) {
   if (a.K <= 0) fail("physics launch: K must be positive");
+  if (const int per_wave = resident_worlds(E)) {
+    ResidentArgs ra{};
+    ra.ph = a;
+    launch_resident_kernel(ra, false, per_wave == 2);
+    HIPCHECK(hipGetLastError());
+    return;
+  }
   chunk_schedule(a, E->pgrid);
   const long per_pair = (long)(a.K - 1) * a.nch + a.nchl;
   if (per_pair > (1L << 30)) fail("physics launch: too many work items per pair");
@@ -840,17 +859,6 @@ static void pack_wide(EnvState* E, const float* W, const float* mean, const floa
   HIPCHECK(hipGetLastError());
 }
 
-// Worlds per wave of the resident form (k_resident), or 0 where the work queue runs the rollout: one while
-// every wave can have a SIMD to itself (1024 worlds), two while all waves are resident at once (4096).
-// Measured, ms per 32 steps of the 256-256 policy with one world per wave, two, and the queue: 1024
-// worlds 3.38, 3.85, 5.42; 1536 3.86, 3.87, 5.48; 2048 3.99, 3.81, 5.51; 4096 -, 4.46, 6.02; past that
-// a second round of waves would start when the first ends, and the queue spreads the work evenly (8192
-// worlds 7.6). An env set to the fenced hand-over keeps the queue, which that mode is about.
-static int resident_worlds(const EnvState* E) {
-  if (E->fences) return 0;
-  return E->N <= E->waves / 2 ? 1 : (E->N <= 2 * E->waves ? 2 : 0);
-}
-
 // The whole rollout as one k_resident launch on the null stream; wp as in rollout_fused.
 static void rollout_resident(EnvState* E, int per_wave, int H, const float* W, const float* mean, const float* var,
                              float* O, float* A, float* LP, float* V, float* R, float* D, float* Vlast,
@@ -865,7 +873,7 @@ static void rollout_resident(EnvState* E, int per_wave, int H, const float* W, c
   ra.po = TileArgs{Wt, TileLayout{}, act_noise, O, A, LP, V, Vlast, H, 1, wl, nullptr};
   const bool prof = E->prof_on != 0 && !wp;
   if (prof) prof_mark(E->ev_phys, E->n_phys);
-  launch_resident_kernel(ra, per_wave == 2);
+  launch_resident_kernel(ra, true, per_wave == 2);
   HIPCHECK(hipGetLastError());
   if (prof) prof_mark(E->ev_phys, E->n_phys);
 }

@@ -11,7 +11,8 @@
 // world per wave and 9.5 us with two (a wave alone on its SIMD), the rest of a control step 15 us, of
 // which the 256-256 policy is about 10. Rollouts of 32 control steps against the queue: 32 worlds 4.36 ->
 // 3.11 ms, 1024 5.42 -> 3.38, 2048 5.51 -> 3.81, 4096 6.02 -> 4.46; 512-512-256 policy, 4 steps of 512
-// worlds 1.26 -> 0.67, 8 steps of 4096 2.83 -> 1.81.
+// worlds 1.26 -> 0.67, 8 steps of 4096 2.83 -> 1.81. Control steps on given actions (the host step,
+// g1_env_bench_phys) gain the hand-overs between the queue's four items of a step: 3-4% of a launch.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -300,9 +301,10 @@ __device__ __forceinline__ int finish_control_step(const PhysArgs& a, const Lane
   return d_flag;
 }
 
-// Enqueue k_resident on the null stream (resident_kernel.hip), with two worlds per wave or one.
-void launch_resident_kernel(const ResidentArgs& ra, bool two);
-// k_resident's function handles (occupancy report).
+// Enqueue k_resident on the null stream (resident_kernel.hip), with two worlds per wave or one: the
+// policy's rollout of ra.ph.K control steps, or (policy false) K >= 1 control steps on ra.ph.act.
+void launch_resident_kernel(const ResidentArgs& ra, bool policy, bool two);
+// The rollout's function handles (occupancy report).
 const void* resident_kernel_fn(bool two);
 
 }  // namespace g1k

@@ -1,5 +1,5 @@
-// resident_kernel.hip -- k_resident, a whole rollout with one or two worlds per wave (resident.h). Its own
-// translation unit for the wavefront-fence phase boundaries.
+// resident_kernel.hip -- k_resident: a whole rollout, or K control steps on given actions, with one or two
+// worlds per wave (resident.h). Its own translation unit for the wavefront-fence phase boundaries.
 #include <hip/hip_runtime.h>
 
 #define G1_PHASE_FENCE   // world_qacc's phase boundaries as wavefront fences (see wave_sync)
@@ -10,7 +10,8 @@ namespace g1k {
 // kW: worlds per wave. With two, group g of block b has world 2 b + g; with one, both groups carry world
 // b and group 0 stores: the second group costs nothing (its lanes would idle), and the wave then runs
 // the contact phases at its own world's contact count instead of the larger of two.
-template <int kW>
+// kPolicy: the actions come from the policy (K = H steps), else from ph.act.
+template <int kW, bool kPolicy>
 __global__ void __launch_bounds__(kPhysThreads) k_resident(ResidentArgs ra) {
   __shared__ __align__(16) WorldLds lds[2];
   const int g = group_id(), l = group_lane();
@@ -43,23 +44,28 @@ __global__ void __launch_bounds__(kPhysThreads) k_resident(ResidentArgs ra) {
 #pragma unroll 1
   for (int k = 0;; ++k) {
     const ResidentArgs& rb = kernarg_reread<ResidentArgs>();
-    const float act =
-        wave_policy<kW>(rb.po, st, pa, rng, rb.ph.seed, rb.ph.N, k, w, wc, wvalid, reinterpret_cast<float*>(lds));
-    if (k >= K) break;   // the bootstrap value of the state after the last step
+    float act = 0.f;
+    if (kPolicy)   // k == K: the bootstrap value of the state after the last step
+      act = wave_policy<kW>(rb.po, st, pa, rng, rb.ph.seed, rb.ph.N, k, w, wc, wvalid, reinterpret_cast<float*>(lds));
+    if (k >= K) break;
     // the lane's model constants, formed here (opaque lane index) rather than held across steps
     int lo = l;
     __asm__ volatile("" : "+v"(lo));
     const LaneModel L = lane_model(lo);
     const PhysArgs& a = kernarg_reread<ResidentArgs>().ph;
+    const int t = a.t0 + k * a.astep;
+    if (!kPolicy) act = hinge ? a.act[((long)t * a.N + wc) * kAct + l - 2] : 0.f;
     float vx_sum = 0.f, energy = 0.f;
     const SolveParams P{a.pgs, a.mu, true, true};
     run_substeps(P, s, L, l, wvalid, pd_target(L, act), 0, a.S, st, energy, vx_sum, hcnt);
     float r;
-    const int done = finish_control_step(a, L, l, wc, k, act, vx_sum, energy, st, pa, step, rng, r);
+    const int done = finish_control_step(a, L, l, wc, t, act, vx_sum, energy, st, pa, step, rng, r);
     if (wvalid && l == 1) {
-      a.R[(long)k * a.N + w] = r;
-      a.D[(long)k * a.N + w] = (float)done;
+      const long o = (long)(a.t0 + k * a.rstep) * a.N + w;
+      a.R[o] = r;
+      a.D[o] = (float)done;
     }
+    if (!kPolicy && k == K - 1 && a.obs && wvalid) store_observation(a.obs + (long)w * kObs, L, l, st, pa);
   }
   const PhysArgs& a = kernarg_reread<ResidentArgs>().ph;
   if (wvalid && a.K > 0) {
@@ -74,11 +80,16 @@ __global__ void __launch_bounds__(kPhysThreads) k_resident(ResidentArgs ra) {
   if (a.ncon_hist && l < 9 && hcnt) atomicAdd(&a.ncon_hist[l], (unsigned long long)hcnt);
 }
 
-void launch_resident_kernel(const ResidentArgs& ra, bool two) {
-  if (two) hipLaunchKernelGGL(k_resident<2>, dim3((unsigned)(ra.ph.N + 1) / 2), dim3(kPhysThreads), 0, 0, ra);
-  else hipLaunchKernelGGL(k_resident<1>, dim3((unsigned)ra.ph.N), dim3(kPhysThreads), 0, 0, ra);
+void launch_resident_kernel(const ResidentArgs& ra, bool policy, bool two) {
+  const dim3 grid((unsigned)(two ? (ra.ph.N + 1) / 2 : ra.ph.N)), block(kPhysThreads);
+  if (policy && two) hipLaunchKernelGGL((k_resident<2, true>), grid, block, 0, 0, ra);
+  else if (policy) hipLaunchKernelGGL((k_resident<1, true>), grid, block, 0, 0, ra);
+  else if (two) hipLaunchKernelGGL((k_resident<2, false>), grid, block, 0, 0, ra);
+  else hipLaunchKernelGGL((k_resident<1, false>), grid, block, 0, 0, ra);
 }
 
-const void* resident_kernel_fn(bool two) { return two ? (const void*)k_resident<2> : (const void*)k_resident<1>; }
+const void* resident_kernel_fn(bool two) {
+  return two ? (const void*)k_resident<2, true> : (const void*)k_resident<1, true>;
+}
 
 }  // namespace g1k

@@ -1,5 +1,5 @@
-"""Rollouts of batches that fit the chip at one or two worlds per wave (k_resident, up to 4096 worlds) against
-the work-queue form (k_rollout), which the fenced hand-over keeps at every size: every trajectory output, the
+"""Launches on batches that fit the chip at one or two worlds per wave (k_resident, up to 4096 worlds) against
+the work-queue form (k_rollout, k_physics), which the fenced hand-over keeps at every size: every output, the
 final state and the contact histogram bit for bit. The two forms share the physics, and the policy's sums run
 in the same order on the vector ALUs as on v_mfma_f32_16x16x4f32, so the tolerance is zero."""
 import numpy as np
@@ -60,3 +60,27 @@ def test_resident_rollout_equals_work_queue(g1, N, H, S, hidden, act, given):
     for i, (a, b) in enumerate(zip(*got)):
         assert np.array_equal(a, b), i
     assert H == 0 or (got[0][5] != 0).any()   # some world finished
+
+
+@pytest.mark.parametrize("N,S", [(1, 10), (33, 1), (1024, 5), (1025, 4), (4095, 3)])
+def test_resident_control_steps_equal_work_queue(g1, N, S):
+    """Host steps (observation, reward, done; a finished world restarts) and zero-action physics: the two forms'
+    outputs and states bit for bit."""
+    import configs
+    rng = np.random.default_rng(N)
+    qp, qv, pa, steps = configs.reset_states(rng, N, noise=0.1)
+    qv = rng.normal(0, 0.3, qv.shape).astype(np.float32)
+    steps[::3] = 998
+    acts = rng.normal(0, 0.5, (3, N, 29)).astype(np.float32)
+    got = []
+    for fences in (0, 1):
+        with g1.Env(N, substeps=S, pgs_iters=8, seed=4) as env:
+            env.set_handover(fences)
+            env.set_state(qp, qv, pa, steps)
+            env.ncon_hist(enable=True)
+            out = [x for a in acts for x in env.step(a)]
+            env.bench_phys(2)
+            got.append([x.view(np.uint32) for x in out + list(env.get_state())] + [env.ncon_hist(enable=False)])
+            assert env.check() == 0
+    for i, (a, b) in enumerate(zip(*got)):
+        assert np.array_equal(a, b), i
