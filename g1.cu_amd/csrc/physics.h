@@ -478,40 +478,63 @@ struct SolveParams {
 // fma (v_fmac_f32 with a DPP source operand): 4 VALU. Written out because the compiler keeps the
 // DPP move apart from an fma (it forms the two-operand v_fmac_f32 only after its DPP combining)
 // and, with the fma written out alone, adds a canonicalising max before max(-r, 0); these are the
-// compiler's own instructions for the operations, so the values are the same. The s_nop and the
-// v_cndmask before the DPP read give the two wait states it needs after the VALU write of its
-// source. max(-r, 0) is 0 for a NaN r (the quiet NaNs of arithmetic), as t > 0 ? t : 0 is.
-// `lanes`: the row's lanes, lane II of every 16-lane row (a mask built from an opaque base in each
-// sweep: as 32 constants the compiler holds the masks in scalar registers across the sweep loop
-// and spills them).
-template <int II, int W>
-__device__ __forceinline__ void pgs_row(float a, int l, unsigned long long lanes, float& fi, float& ri) {
-  static_assert(W == 4 || W == 16, "rows of a quad or of a 16-lane row");
-  if constexpr (W == 4) {
-    const float t = -ri;
-    const float fn = t > 0.f ? t : 0.f;
-    const float d = fn - fi;
-    fi = (l == II) ? fn : fi;
-    ri = fmaf_(a, group_bcast<II, W>(d), ri);
-  } else {
-    float fn, d;
-    __asm__("v_max_f32_e64 %2, -%1, 0\n\t"
-            "v_sub_f32_e32 %3, %2, %0\n\t"
-            "v_cndmask_b32_e64 %0, %0, %2, %5\n\t"
-            "s_nop 0\n\t"
-            "v_fmac_f32_dpp %1, %3, %4 row_newbcast:%6 row_mask:0xf bank_mask:0xf"
-            : "+v"(fi), "+v"(ri), "=&v"(fn), "=&v"(d)
-            : "v"(a), "s"(lanes), "n"(II & 15));
-  }
+// compiler's own instructions for the operations, so the values are the same. The four rows of a
+// contact are one block (between blocks of one row the compiler puts an s_nop for a DPP read that it
+// cannot see), and the lane mask moves on to the next row between the two wait states that a DPP read
+// needs after the VALU write of its source, where an s_nop stood: six issue slots per row in the paired
+// form and five in the other, two fewer than a block per row with the mask formed outside (50 steps of
+// 8192 standing worlds 20.79 -> 20.58 ms). max(-r, 0) is 0 for a NaN r (the quiet NaNs of arithmetic), as t > 0 ? t : 0 is.
+// `lanes`: the row's lanes, lane II of every 16-lane row (from an opaque base in each sweep: as 32
+// constants the compiler holds the masks in scalar registers across the sweep loop and spills them).
+
+// Lane 0 of every 16-lane row: the lanes of a sweep's first row.
+__device__ __forceinline__ unsigned long long pgs_lanes0() {
+  unsigned long long lanes = 0x0001000100010001ull;
+  __asm__ volatile("" : "+s"(lanes));
+  return lanes;
 }
 
+// rows II .. II + 3 (II a multiple of 4)
+#define G1_PGS_ROW(A, I)                               \
+  "v_max_f32_e64 %2, -%1, 0\n\t"                       \
+  "v_sub_f32_e32 %3, %2, %0\n\t"                       \
+  "v_cndmask_b32_e64 %0, %0, %2, %4\n\t"               \
+  "s_lshl_b64 %4, %4, 1\n\t"                           \
+  "v_fmac_f32_dpp %1, %3, " A " row_newbcast:" I " row_mask:0xf bank_mask:0xf\n\t"
 template <int II, int W>
-__device__ __forceinline__ void pgs_sweep(const float (&Acol)[kMaxEfc], int l, unsigned long long lanes0, int nefc_max,
+__device__ __forceinline__ void pgs_rows(const float (&A)[kMaxEfc], int l, unsigned long long& lanes, float& fi,
+                                         float& ri) {
+  static_assert(W == 4 || W == 16, "rows of a quad or of a 16-lane row");
+  if constexpr (W == 4) {
+    auto row = [&](auto k) {
+      constexpr int I = decltype(k)::value;
+      const float t = -ri;
+      const float fn = t > 0.f ? t : 0.f;
+      const float d = fn - fi;
+      fi = (l == I) ? fn : fi;
+      ri = fmaf_(A[I], group_bcast<I, W>(d), ri);
+    };
+    row(std::integral_constant<int, II>());
+    row(std::integral_constant<int, II + 1>());
+    row(std::integral_constant<int, II + 2>());
+    row(std::integral_constant<int, II + 3>());
+  } else {
+    float fn, d;
+    __asm__(G1_PGS_ROW("%5", "%9") G1_PGS_ROW("%6", "%10") G1_PGS_ROW("%7", "%11") G1_PGS_ROW("%8", "%12")
+            : "+v"(fi), "+v"(ri), "=&v"(fn), "=&v"(d), "+s"(lanes)
+            : "v"(A[II]), "v"(A[II + 1]), "v"(A[II + 2]), "v"(A[II + 3]), "n"(II), "n"(II + 1), "n"(II + 2), "n"(II + 3)
+            : "scc");
+  }
+}
+#undef G1_PGS_ROW
+
+template <int II, int W>
+__device__ __forceinline__ void pgs_sweep(const float (&Acol)[kMaxEfc], int l, unsigned long long lanes, int nefc_max,
                                           float& fi, float& ri) {
   if constexpr (II < W) {
-    if (II % 4 != 0 || II < nefc_max) {
-      pgs_row<II, W>(Acol[II], l, lanes0 << II, fi, ri);
-      pgs_sweep<II + 1, W>(Acol, l, lanes0, nefc_max, fi, ri);
+    if (II < nefc_max) {
+      pgs_rows<II, W>(Acol, l, lanes, fi, ri);
+      pgs_sweep<II + 4, W>(Acol, l, lanes, nefc_max, fi, ri);
     }
   }
 }
@@ -522,47 +545,41 @@ __device__ __forceinline__ void pgs_sweep(const float (&Acol)[kMaxEfc], int l, u
 // every 16-lane row, so one DPP row_newbcast inside each of the two fmas (r_lo += p_II d,
 // r_hi += q_II d) broadcasts it: 5 VALU per row, where one row per lane needs a cross-row exchange
 // (v_permlane16_swap, its register copy and wait states) on every row. Same operations in the same
-// order as one row per lane, so the same values.
+// order as one row per lane, so the same values. Rows II .. II + 3: A the entries of the rows' own half
+// (p for II < 16), B of the other, r and ro their residuals.
+#define G1_PGS_ROW(A, B, I)                                                          \
+  "v_max_f32_e64 %3, -%1, 0\n\t"                                                     \
+  "v_sub_f32_e32 %4, %3, %0\n\t"                                                     \
+  "v_cndmask_b32_e64 %0, %0, %3, %5\n\t"                                             \
+  "s_lshl_b64 %5, %5, 1\n\t"                                                         \
+  "v_fmac_f32_dpp %1, %4, " A " row_newbcast:" I " row_mask:0xf bank_mask:0xf\n\t"   \
+  "v_fmac_f32_dpp %2, %4, " B " row_newbcast:" I " row_mask:0xf bank_mask:0xf\n\t"
 template <int II>
-__device__ __forceinline__ void pgs_row_pair(float p, float q, unsigned long long lanes, float& fown, float& rlo,
-                                             float& rhi) {
+__device__ __forceinline__ void pgs_rows_pair(const float (&A)[kMaxEfc], const float (&B)[kMaxEfc],
+                                              unsigned long long& lanes, float& f, float& r, float& ro) {
   float fn, d;
-  if constexpr (II < 16) {
-    __asm__("v_max_f32_e64 %3, -%1, 0\n\t"
-            "v_sub_f32_e32 %4, %3, %0\n\t"
-            "v_cndmask_b32_e64 %0, %0, %3, %7\n\t"
-            "s_nop 0\n\t"
-            "v_fmac_f32_dpp %1, %4, %5 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
-            "v_fmac_f32_dpp %2, %4, %6 row_newbcast:%8 row_mask:0xf bank_mask:0xf"
-            : "+v"(fown), "+v"(rlo), "+v"(rhi), "=&v"(fn), "=&v"(d)
-            : "v"(p), "v"(q), "s"(lanes), "n"(II & 15));
-  } else {
-    __asm__("v_max_f32_e64 %3, -%2, 0\n\t"
-            "v_sub_f32_e32 %4, %3, %0\n\t"
-            "v_cndmask_b32_e64 %0, %0, %3, %7\n\t"
-            "s_nop 0\n\t"
-            "v_fmac_f32_dpp %1, %4, %5 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
-            "v_fmac_f32_dpp %2, %4, %6 row_newbcast:%8 row_mask:0xf bank_mask:0xf"
-            : "+v"(fown), "+v"(rlo), "+v"(rhi), "=&v"(fn), "=&v"(d)
-            : "v"(p), "v"(q), "s"(lanes), "n"(II & 15));
-  }
+  __asm__(G1_PGS_ROW("%6", "%10", "%14") G1_PGS_ROW("%7", "%11", "%15") G1_PGS_ROW("%8", "%12", "%16")
+          G1_PGS_ROW("%9", "%13", "%17")
+          : "+v"(f), "+v"(r), "+v"(ro), "=&v"(fn), "=&v"(d), "+s"(lanes)
+          : "v"(A[II]), "v"(A[II + 1]), "v"(A[II + 2]), "v"(A[II + 3]), "v"(B[II]), "v"(B[II + 1]), "v"(B[II + 2]),
+            "v"(B[II + 3]), "n"(II & 15), "n"((II & 15) + 1), "n"((II & 15) + 2), "n"((II & 15) + 3)
+          : "scc");
 }
+#undef G1_PGS_ROW
 
 template <int II>
 __device__ __forceinline__ void pgs_sweep_pair(const float (&P)[kMaxEfc], const float (&Q)[kMaxEfc],
-                                               unsigned long long lanes0, int nefc_max, float& flo, float& fhi,
+                                               unsigned long long lanes, int nefc_max, float& flo, float& fhi,
                                                float& rlo, float& rhi) {
   if constexpr (II < kMaxEfc) {
-    if (II % 4 != 0 || II < nefc_max) {
-      if constexpr (II < 16) pgs_row_pair<II>(P[II], Q[II], lanes0 << II, flo, rlo, rhi);
-      else pgs_row_pair<II>(P[II], Q[II], lanes0 << (II - 16), fhi, rlo, rhi);
-      pgs_sweep_pair<II + 1>(P, Q, lanes0, nefc_max, flo, fhi, rlo, rhi);
+    if (II < nefc_max) {
+      if constexpr (II == 16) lanes = pgs_lanes0();   // the high rows start at lane 0 again
+      if constexpr (II < 16) pgs_rows_pair<II>(P, Q, lanes, flo, rlo, rhi);
+      else pgs_rows_pair<II>(Q, P, lanes, fhi, rhi, rlo);
+      pgs_sweep_pair<II + 4>(P, Q, lanes, nefc_max, flo, fhi, rlo, rhi);
     }
   }
 }
-
-// Lane 0 of every 16-lane row: the row lanes of a sweep's first row (pgs_row, pgs_row_pair).
-constexpr unsigned long long kPgsLanes0 = 0x0001000100010001ull;
 
 // Sweeps between the fresh residuals of the PGS (a fresh residual r_i = c_i + sum_k a_ik f_k, k in
 // order, bounds the rounding the row updates carry over long solves).
@@ -1802,9 +1819,7 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
         ri = done ? ri : t;
       }
       const float f0 = fi;
-      unsigned long long lanes0 = kPgsLanes0;
-      __asm__ volatile("" : "+s"(lanes0));
-      pgs_sweep<0, W>(Acol, l, lanes0, nefc_max, fi, ri);
+      pgs_sweep<0, W>(Acol, l, pgs_lanes0(), nefc_max, fi, ri);
       const unsigned long long m = __ballot(__float_as_uint(fi) != __float_as_uint(f0));
       if (m == 0ull) break;
       done = done || ((unsigned)(m >> (32 * group_id())) == 0u);
@@ -1850,9 +1865,7 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
         rhi = done ? rhi : thi;
       }
       const float flo0 = flo, fhi0 = fhi;
-      unsigned long long lanes0 = kPgsLanes0;
-      __asm__ volatile("" : "+s"(lanes0));
-      pgs_sweep_pair<0>(Pr, Qr, lanes0, nefc_max, flo, fhi, rlo, rhi);
+      pgs_sweep_pair<0>(Pr, Qr, pgs_lanes0(), nefc_max, flo, fhi, rlo, rhi);
       const unsigned long long m = __ballot(__float_as_uint(flo) != __float_as_uint(flo0) ||
                                             __float_as_uint(fhi) != __float_as_uint(fhi0));
       if (m == 0ull) break;
