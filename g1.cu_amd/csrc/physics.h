@@ -316,7 +316,9 @@ struct WorldLds {
       alignas(16) float Dinv[6];        // RN(1 / diagonal of Dfac)
       alignas(16) float Dm[36];         // free-joint 6x6 block before factoring
     } fac;
-    alignas(16) float G[kPairs][9];     // 3x3 Gram blocks of contact pairs c <= c' (after the solves)
+    // 3x3 Gram blocks of contact pairs c <= c' (after the solves), row a of the block four floats at
+    // G[0][pair][a], and the transposed blocks in G[1]; the last block of G[0] holds zeros
+    alignas(16) float G[2][kPairs + 1][3][4];
   } u;
   alignas(16) float qvel[kNV + 1];
   union {
@@ -1687,8 +1689,10 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
     }
     if (blk) {
       const int pr = cp * (cp + 1) / 2 + c;
-      s.u.G[pr][0 * 3 + bcol] = g0; s.u.G[pr][1 * 3 + bcol] = g1; s.u.G[pr][2 * 3 + bcol] = g2;
+      s.u.G[0][pr][0][bcol] = g0; s.u.G[0][pr][1][bcol] = g1; s.u.G[0][pr][2][bcol] = g2;
+      s.u.G[1][pr][bcol][0] = g0; s.u.G[1][pr][bcol][1] = g1; s.u.G[1][pr][bcol][2] = g2;
     }
+    if (l < 12) (&s.u.G[0][kPairs][0][0])[l] = 0.f;
     if (bvc) {
       s.bvec[4 * c + 0] = fmaf_(0.f, g2, fmaf_(1.f, g1, 1.f * g0)) - s.aref[4 * c + 0];
       s.bvec[4 * c + 1] = fmaf_(0.f, g2, fmaf_(-1.f, g1, 1.f * g0)) - s.aref[4 * c + 1];
@@ -1730,10 +1734,12 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
             g0 = fmaf_(s.Eb[c][0][k], mv, g0); g1 = fmaf_(s.Eb[c][1][k], mv, g1); g2 = fmaf_(s.Eb[c][2][k], mv, g2);
           }
           const int pr = cp * (cp + 1) / 2 + c;
-          s.u.G[pr][0 * 3 + bcol] = g0; s.u.G[pr][1 * 3 + bcol] = g1; s.u.G[pr][2 * 3 + bcol] = g2;
+          s.u.G[0][pr][0][bcol] = g0; s.u.G[0][pr][1][bcol] = g1; s.u.G[0][pr][2][bcol] = g2;
+          s.u.G[1][pr][bcol][0] = g0; s.u.G[1][pr][bcol][1] = g1; s.u.G[1][pr][bcol][2] = g2;
         }
       }
     }
+    if (l < 12) (&s.u.G[0][kPairs][0][0])[l] = 0.f;
     if (l < ncon) {
       s.bvec[4 * l + 0] = fmaf_(0.f, bb2, fmaf_(1.f, bb1, 1.f * bb0)) - s.aref[4 * l + 0];
       s.bvec[4 * l + 1] = fmaf_(0.f, bb2, fmaf_(-1.f, bb1, 1.f * bb0)) - s.aref[4 * l + 1];
@@ -1747,47 +1753,70 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
   // directions d0=(1,1,0) d1=(1,-1,0) d2=(1,0,1) d3=(1,0,-1). For a pair c < c' the reference
   // expands d_k' G[c][c'] d_k'' once and mirrors it; within one contact it keeps the value
   // computed with (k, k') = (larger, smaller).
+  // A direction is basis 0 plus or minus basis x (x = 1 for k < 2, else 2), so an entry is two lines of
+  // its 3x3 block and two additions: (G00 + s Gx0) + s' (G0x' + s Gxx') for the lower contact's
+  // direction (x, s) and the higher one's (x', s') (the reference's products with the directions'
+  // zeros and ones are exact). A lane takes line 0 and line x of its own direction, p and q, as two
+  // 16-byte reads: rows of the block where its contact is the lower one (c2 > ci: the own sum p + s q
+  // comes first, for all four columns), of the transposed block where it is the higher one. With a
+  // 9-float read and the general products and selects per entry 50 steps of 8192 standing worlds took
+  // 20.58 ms, now 20.05; 8192 contact solves 44.9 -> 44.2 us.
   const int nefc = 4 * ncon, nefc_max = 4 * ncon_max;
   const int ci = l >> 2, ki = l & 3;
   const bool row = l < nefc;
-  auto dcoef = [](int k, int a) -> float {
-    return a == 0 ? 1.f : (a == 1 ? (k == 0 ? 1.f : (k == 1 ? -1.f : 0.f)) : (k == 2 ? 1.f : (k == 3 ? -1.f : 0.f)));
+  const float sk = (ki & 1) ? -1.f : 1.f;   // the lane's own direction: sign s and line x
+  const int xk = ki < 2 ? 1 : 2;
+  // the entries of the pair whose lines are p and q, for the other contact's four directions: `up`
+  // where the lane's contact is the lower one
+  auto up = [&](const float4& p, const float4& q, float (&v)[4]) {
+    const float t0 = fmaf_(sk, q.x, p.x), t1 = fmaf_(sk, q.y, p.y), t2 = fmaf_(sk, q.z, p.z);
+    v[0] = t0 + t1; v[1] = t0 - t1; v[2] = t0 + t2; v[3] = t0 - t2;
   };
-  // Entries are formed by every lane (branch-free; the G block and R indices stay inside their
-  // arrays for every lane) and kept where (row, column) is a constraint pair; the row loop stops at
-  // the wave's largest row count.
+  auto down = [&](const float4& p, const float4& q, float (&v)[4]) {
+    v[0] = fmaf_(sk, q.x + q.y, p.x + p.y); v[1] = fmaf_(sk, q.x - q.y, p.x - p.y);
+    v[2] = fmaf_(sk, q.x + q.z, p.x + p.z); v[3] = fmaf_(sk, q.x - q.z, p.x - p.z);
+  };
+  auto lines = [&](const float* blk, float4& p, float4& q) {
+    p = *reinterpret_cast<const float4*>(blk);
+    q = *reinterpret_cast<const float4*>(blk + 4 * xk);
+  };
+  const float* const G0 = &s.u.G[0][0][0][0];
+  const float* const G1 = &s.u.G[1][0][0][0];
+  const float* const Gz = &s.u.G[0][kPairs][0][0];
+  const int tri = ci * (ci + 1) / 2;
+  // the lane's own contact first: its diagonal entry apart (1 on lanes without a row)
+  float ev[4], Aii;
+  {
+    float4 p, q, pt, qt;
+    lines(row ? G0 + 12 * (tri + ci) : Gz, p, q);
+    lines(row ? G1 + 12 * (tri + ci) : Gz, pt, qt);
+    float dn[4];
+    up(p, q, ev);
+    down(pt, qt, dn);
+    float d = 0.f;
+#pragma unroll
+    for (int k2 = 0; k2 < 4; ++k2) {
+      d = k2 == ki ? ev[k2] : d;
+      ev[k2] = k2 < ki ? ev[k2] : (k2 == ki ? 0.f : dn[k2]);
+    }
+    Aii = row ? d + s.Rc[ci] : 1.f;
+  }
   float Acol[kMaxEfc];
 #pragma unroll
   for (int ii = 0; ii < kMaxEfc; ++ii) Acol[ii] = 0.f;
-  float Aii = 1.f;   // the lane's diagonal entry, taken as it is formed (1 on lanes without a row)
-  const float Rci = s.Rc[ci];
-  // pyramid coefficients of the lane's own row (d0 = 1 for every direction)
-  const float dki1 = dcoef(ki, 1), dki2 = dcoef(ki, 2);
 #pragma unroll
   for (int c2 = 0; c2 < kNFoot; ++c2) {
     if (c2 >= ncon_max) continue;
-    const int lo = c2 < ci ? c2 : ci, hi = c2 < ci ? ci : c2;
-    const float* Gp = s.u.G[hi * (hi + 1) / 2 + lo];
-    float G[9];
+    const bool lt = c2 < ci, eq = c2 == ci;
+    const float* blk = lt ? G1 + 12 * (tri + c2) : G0 + 12 * (c2 * (c2 + 1) / 2 + ci);
+    blk = row && c2 < ncon ? blk : Gz;   // entries outside the world's rows are zero
+    float4 p, q;
+    lines(blk, p, q);
+    float vu[4], vd[4];
+    up(p, q, vu);
+    down(p, q, vd);
 #pragma unroll
-    for (int e = 0; e < 9; ++e) G[e] = Gp[e];
-    const bool lt = c2 < ci, eq = c2 == ci, keep = row && c2 < ncon;
-#pragma unroll
-    for (int k2 = 0; k2 < 4; ++k2) {
-      // (klo, khi) = (k2, ki) if c2 < ci, (ki, k2) if c2 > ci, (max, min) within one contact
-      const bool k2lo = lt || (eq && k2 >= ki);
-      const float dk1 = dcoef(k2, 1), dk2 = dcoef(k2, 2);
-      const float dl1 = k2lo ? dk1 : dki1, dl2 = k2lo ? dk2 : dki2;
-      const float dh1 = k2lo ? dki1 : dk1, dh2 = k2lo ? dki2 : dk2;
-      const float t0 = fmaf_(dl2, G[6], fmaf_(dl1, G[3], 1.f * G[0]));
-      const float t1 = fmaf_(dl2, G[7], fmaf_(dl1, G[4], 1.f * G[1]));
-      const float t2 = fmaf_(dl2, G[8], fmaf_(dl1, G[5], 1.f * G[2]));
-      float val = fmaf_(t2, dh2, fmaf_(t1, dh1, t0 * 1.f));
-      const bool diag = eq && k2 == ki;
-      val = diag ? val + Rci : val;
-      Acol[4 * c2 + k2] = (keep && !diag) ? val : 0.f;   // the diagonal is held apart (Aii)
-      Aii = (diag && row) ? val : Aii;
-    }
+    for (int k2 = 0; k2 < 4; ++k2) Acol[4 * c2 + k2] = eq ? ev[k2] : (lt ? vd[k2] : vu[k2]);
   }
   const float bi = row ? s.bvec[l] : 0.f;
 
