@@ -1552,70 +1552,53 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
     const bool basis = (j >= 1) && (j < kCols) && (cj < ncon);
     const bool right = s.con_leg[cj] != 0;
     const float* eb = s.Eb[cj][aj];
-    // right-hand side entry of dof d, read on demand: the contact basis row e_{c,a} on its 12
-    // ancestor dofs, 0 elsewhere and for idle lanes
-    auto xrhs = [&](int d) -> float {
-      if (d < 6) return basis ? eb[6 + d] : 0.f;
-      if (d < 12) return (basis && !right) ? eb[11 - d] : 0.f;
-      if (d < 18) return (basis && right) ? eb[17 - d] : 0.f;
-      return 0.f;
-    };
-    // leaf -> root. The basis right-hand sides live on the base and leg dofs (the feet hang off
-    // bodies 7 and 13, legs 2..13), so the waist/arm subtree (bodies 14..30) carries zero
-    // articulated bias: u = 0 - S.0 = +0 and its contribution to the pelvis is +0; skipping it
-    // changes no bit. The two legs are independent chains and are walked interleaved (right leg
-    // 13..8 with left leg 7..2) so their dependency chains overlap; the pelvis then adds the
-    // right leg's root (8) before the left leg's (2), the reference's descending order.
+    // leaf -> root. The basis right-hand sides live on the base and the dofs of their own contact's leg
+    // (the feet hang off bodies 7 and 13): the other leg and the waist/arm subtree (bodies 14..30) carry
+    // zero articulated bias (u = 0 - S.0 = +0, and a contribution of +0 to the pelvis). So each lane
+    // walks the leg of its own contact, body d + loff at depth d, 7..2: six levels for all columns.
     static_assert(foot_body[0] < 14 && foot_body[kNFoot - 1] < 14 && body_parent[14] == 1, "leg layout");
     static_assert(body_parent[2] == 1 && body_parent[8] == 1 && body_nchild[7] == 0 && body_nchild[13] == 0, "legs");
-    float u[kNBody];
-#pragma unroll
-    for (int b = 14; b < kNBody; ++b) u[b] = 0.f;
-    // Each body's LDS operands are read one body ahead (`nxt`) so their latency overlaps the
-    // current body's arithmetic; the pin keeps the reads from running further ahead.
-    // (only plain loads: a value used before the pin would make it wait for them)
-    struct UpIn { float S[6], U[6], iD, e; };
-    auto ld_up = [&](int b, UpIn& f) {
-#pragma unroll
-      for (int k = 0; k < 6; ++k) { f.S[k] = s.u.fac.S[b + 4][k]; f.U[k] = s.u.fac.U[b][k]; }
-      f.iD = s.u.fac.U[b][kInvD];
-      f.e = eb[b < 8 ? 7 - b : 13 - b];   // xrhs(b + 4) before its select
-    };
-    constexpr int kUpOrder[12] = {13, 7, 12, 6, 11, 5, 10, 4, 9, 3, 8, 2};
-    float car[2][6] = {}, croot[2][6];   // [0] right leg (13..8), [1] left leg (7..2)
-    UpIn cur, nxt;
-    ld_up(kUpOrder[0], cur);
-#pragma unroll
-    for (int i = 0; i < 12; ++i) {
-      const int b = kUpOrder[i], g = i & 1;
-      if (i + 1 < 12) ld_up(kUpOrder[i + 1], nxt);
-      float pb[6];
-#pragma unroll
-      for (int k = 0; k < 6; ++k) pb[k] = body_nchild[b] == 0 ? 0.f : car[g][k];
-      const bool own = basis && (b < 8 ? !right : right);
-      const float ub = (own ? cur.e : 0.f) - dot6(cur.S, pb);
-      u[b] = ub;
-      const float ud = ub * cur.iD;
-#pragma unroll
-      for (int k = 0; k < 6; ++k) {
-        const float c = fmaf_(cur.U[k], ud, pb[k]);
-        if (body_parent[b] == 1) croot[g][k] = c;
-        else car[g][k] = c;
-      }
-      G1_PIN6(car[g]);
-      __asm__ volatile("" : "+v"(u[b]));
-      if (i + 1 < 12) cur = nxt;
-    }
-    const float (&c8)[6] = croot[0];
-    const float (&c2)[6] = croot[1];
-    float p1[6];
     const bool smooth = j == 0;
+    float ul[6];   // u of the own leg's bodies at depth 2..7
+    float p1[6];
+    {
+      const int loff = right ? 6 : 0;
+      const float* const pS = &s.u.fac.S[loff + 4][0];
+      const float* const pU = &s.u.fac.U[loff][0];
+      float car[6];
+      // Each level's LDS operands are read one level ahead so their latency overlaps the arithmetic;
+      // the pin keeps the reads from running further ahead.
+      float nS[6], nU[6], nD, nE;
+      auto ld = [&](int d) {
 #pragma unroll
-    for (int k = 0; k < 6; ++k) p1[k] = smooth ? pAs[k] : c8[k] + c2[k];
+        for (int k = 0; k < 6; ++k) { nS[k] = pS[kRow * d + k]; nU[k] = pU[kRow * d + k]; }
+        nD = pU[kRow * d + kInvD];
+        nE = eb[7 - d];   // the basis row's entry of dof d + loff + 4 (both legs: entry 7 - d)
+      };
+      ld(7);
+#pragma unroll
+      for (int d = 7; d >= 2; --d) {
+        float Sd[6], Ud[6], pb[6];
+#pragma unroll
+        for (int k = 0; k < 6; ++k) { Sd[k] = nS[k]; Ud[k] = nU[k]; pb[k] = d == 7 ? 0.f : car[k]; }
+        const float iD = nD, e = nE;
+        if (d > 2) ld(d - 1);
+        const float ub = (basis ? e : 0.f) - dot6(Sd, pb);
+        ul[d - 2] = ub;
+        const float ud = ub * iD;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) car[k] = fmaf_(Ud[k], ud, pb[k]);
+        G1_PIN6(car);
+        __asm__ volatile("" : "+v"(ul[d - 2]));
+      }
+      // the pelvis adds the right leg's root, then the left's; the other one's is +0
+#pragma unroll
+      for (int k = 0; k < 6; ++k) p1[k] = smooth ? pAs[k] : car[k] + 0.f;
+    }
     // free joint: D qdd = x_base - S_base.pA_1 with D = L L'
     float qdd[6], a1[6], xbj[6];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) xbj[k] = smooth ? xb0[k] : xrhs(k);
+    for (int k = 0; k < 6; ++k) xbj[k] = smooth ? xb0[k] : (basis ? eb[6 + k] : 0.f);
     base_solve(s, xbj, p1, qdd, a1);
     float* ycol = s.Mm[j < kCols ? j : kCols - 1];
     const bool wr = j < kCols;
@@ -1648,7 +1631,9 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
       float ap[6];
 #pragma unroll
       for (int k = 0; k < 6; ++k) ap[k] = body_parent[b] == 1 ? a1[k] : body_parent[b] == 16 ? acc[2][k] : acc[ch][k];
-      const float q = ((smooth ? dc.us : u[b]) - dot6(dc.U, ap)) * dc.iD;
+      // u: the smooth solve's, the own leg's from above, +0 elsewhere
+      const float u = b < 14 && right == (b >= 8) ? ul[b < 14 ? body_depth[b] - 2 : 0] : 0.f;
+      const float q = ((smooth ? dc.us : u) - dot6(dc.U, ap)) * dc.iD;
       if (wr) ycol[b + 4] = q;
 #pragma unroll
       for (int k = 0; k < 6; ++k) acc[ch][k] = fmaf_(dc.S[k], q, ap[k]);
