@@ -555,10 +555,13 @@ struct EnvState {
   float *qp, *qv, *pa;
   int* steps;
   unsigned* rng;
-  float *dact, *zero_act, *bench_r, *bench_d;
-  float* dout;            // host-step outputs on the device: [obs N x 100 | reward N | done N]
-  float *h_act, *h_out;   // pinned host staging of the host-step path: actions in; obs, reward, done, queue error out
-  hipEvent_t step_ev[kStepChunks + 1];   // host-step output copies done: observation chunks, reward/done
+  float *zero_act, *bench_r, *bench_d;
+  // host-step path: pinned host memory that the kernels read (actions) and, for small batches, write
+  // ([obs N x 100 | reward N | done N]); for large ones the outputs on the device, and the events of
+  // their copies (observation chunks, reward/done)
+  float *h_act, *h_out;
+  float* dout;
+  hipEvent_t step_ev[kStepChunks + 1];
   float* Wp;
   long Wp_cap;
   unsigned long long* ncon_hist;
@@ -566,7 +569,7 @@ struct EnvState {
   // physics work queue (k_physics): per-pair item flags, claim counters, split-step accumulators
   unsigned* qflags;
   unsigned* qctr;
-  int* qerr;
+  int* qerr;        // the error word, in pinned host memory (only ever stored to on the device)
   float *qacc_e, *qacc_vx;
   unsigned qdone;   // value of every pair flag after the launches enqueued so far
   int qpar;         // counter row of the next launch
@@ -585,7 +588,6 @@ struct EnvState {
   long Wt_cap;
   float* scr;       // wide one-launch policy: per block two activation buffers (WideLayout::maxT * 256 floats each)
   long scr_cap;
-  int* h_qerr;      // pinned copy of qerr, refreshed asynchronously after every rollout
   // per-launch HIP events of the rollout's physics / policy kernels (null stream)
   int prof_on;
   std::vector<hipEvent_t> ev_phys, ev_pol;
@@ -803,19 +805,11 @@ static void check_queue_error(int err) {
   if (err) fail("physics work queue: a block ran outside the XCD its queue was placed on");
 }
 
-static void check_queue(EnvState* E) {
-  int err = 0;
-  HIPCHECK(hipMemcpy(&err, E->qerr, sizeof(int), hipMemcpyDeviceToHost));
-  check_queue_error(err);
-}
-
-// The asynchronous entry points (g1_rollout*) end with a copy of the error word into pinned host
-// memory; every later entry reads that copy without synchronising, so an error stops the caller at
-// its next call into the library once the copy has landed (and at the latest in g1_env_destroy or
-// at the next synchronising call, which read the device word itself).
-static void poll_queue_error(EnvState* E) {
-  check_queue_error(*(volatile int*)E->h_qerr);
-}
+// Reads the word as it stands. The device writes it through to host memory, so after a synchronisation
+// it is the launches' own; the asynchronous entry points (g1_rollout*) do not wait, and an error of
+// theirs stops the caller at a later entry (at the latest in g1_env_destroy or at the next
+// synchronising call).
+static void check_queue(EnvState* E) { check_queue_error(*(volatile int*)E->qerr); }
 
 // The one-launch rollout runs policies of two hidden layers of at most 256 units each on the
 // register-resident tile (policy_tile, at 256-256 with zero padding) and every other accepted shape
@@ -926,13 +920,12 @@ static void rollout_fused(EnvState* E, int H, const float* W, const float* mean,
   E->qdone += H > 0 ? (unsigned)((H - 1) * a.nch + a.nchl) : 0u;
   E->tdone += (unsigned)H + 1u;
   E->qpar ^= 1;
-  HIPCHECK(hipMemcpyAsync(E->h_qerr, E->qerr, sizeof(int), hipMemcpyDeviceToHost, 0));
 }
 
 static void rollout_impl(EnvState* E, int H, const float* W, const float* mean, const float* var, float* O, float* A,
                          float* LP, float* V, float* R, float* D, float* Vlast, const float* act_noise,
                          const float* reset_noise, float* wp = nullptr, long wp_cap = 0) {
-  poll_queue_error(E);
+  check_queue(E);
   if (H < 0) H = 0;   // no control step; the bootstrap value is still computed (as the reference's k_rollout)
   if (E->fused && fused_shape(E->shape, wp != nullptr)) {
     if (const int per_wave = resident_worlds(E)) {
@@ -958,7 +951,6 @@ static void rollout_impl(EnvState* E, int H, const float* W, const float* mean, 
   if (prof) prof_mark(E->ev_pol, E->n_pol);
   launch_policy(E, pp, H, H, mean, var, act_noise, O, A, LP, V, Vlast);
   if (prof) prof_mark(E->ev_pol, E->n_pol);
-  HIPCHECK(hipMemcpyAsync(E->h_qerr, E->qerr, sizeof(int), hipMemcpyDeviceToHost, 0));
 }
 
 // ---- packed policy weights of g1_rollout_noalloc: a file-scope device array, so the entry point
@@ -997,7 +989,6 @@ void* g1_env_create(int N, int substeps, int pgs_iters, unsigned long seed) {
   dev_alloc(E, &E->pa, (size_t)N * kAct * 4);
   dev_alloc(E, &E->steps, (size_t)N * 4);
   dev_alloc(E, &E->rng, (size_t)N * 4);
-  dev_alloc(E, &E->dact, (size_t)N * kAct * 4);
   dev_alloc(E, &E->zero_act, (size_t)N * kAct * 4);
   dev_alloc(E, &E->bench_r, (size_t)N * 4);
   dev_alloc(E, &E->bench_d, (size_t)N * 4);
@@ -1005,12 +996,10 @@ void* g1_env_create(int N, int substeps, int pgs_iters, unsigned long seed) {
   const int npairs = (N + 1) / 2;
   dev_alloc(E, &E->qflags, (size_t)npairs * sizeof(unsigned));
   dev_alloc(E, &E->qctr, 2 * kQueues * sizeof(unsigned));
-  dev_alloc(E, &E->qerr, sizeof(int));
   dev_alloc(E, &E->qacc_e, (size_t)N * kGroup * 4);
   dev_alloc(E, &E->qacc_vx, (size_t)N * 4);
   HIPCHECK(hipMemset(E->qflags, 0, (size_t)npairs * sizeof(unsigned)));
   HIPCHECK(hipMemset(E->qctr, 0, 2 * kQueues * sizeof(unsigned)));
-  HIPCHECK(hipMemset(E->qerr, 0, sizeof(int)));
   E->qdone = 0; E->qpar = 0;
   dev_alloc(E, &E->tflags, (size_t)kQueues * tiles_per_queue(N) * sizeof(unsigned));
   HIPCHECK(hipMemset(E->tflags, 0, (size_t)kQueues * tiles_per_queue(N) * sizeof(unsigned)));
@@ -1046,10 +1035,11 @@ void* g1_env_create(int N, int substeps, int pgs_iters, unsigned long seed) {
       if (hx[b] != b % kXcds) E->xlocal = 0;
   }
   dev_alloc(E, &E->dout, (size_t)N * (kObs + 2) * 4);
-  HIPCHECK(hipHostMalloc((void**)&E->h_act, (size_t)N * kAct * 4, hipHostMallocDefault));
-  HIPCHECK(hipHostMalloc((void**)&E->h_out, ((size_t)N * (kObs + 2) + 1) * 4, hipHostMallocDefault));
-  HIPCHECK(hipHostMalloc((void**)&E->h_qerr, sizeof(int), hipHostMallocDefault));
-  *E->h_qerr = 0;
+  const unsigned shared = hipHostMallocMapped | hipHostMallocCoherent;   // kernels access these directly
+  HIPCHECK(hipHostMalloc((void**)&E->h_act, (size_t)N * kAct * 4, shared));
+  HIPCHECK(hipHostMalloc((void**)&E->h_out, (size_t)N * (kObs + 2) * 4, shared));
+  HIPCHECK(hipHostMalloc((void**)&E->qerr, sizeof(int), shared));
+  *E->qerr = 0;
   for (hipEvent_t& e : E->step_ev) HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   HIPCHECK(hipMemset(E->zero_act, 0, (size_t)N * kAct * 4));
   HIPCHECK(hipMemset(E->rng, 0, (size_t)N * 4));
@@ -1068,76 +1058,95 @@ void g1_env_destroy(void* h) {
   if (!E) return;
   HIPCHECK(hipDeviceSynchronize());
   check_queue(E);
-  void* bufs[] = {E->qp,       E->qv,      E->pa,        E->steps,   E->rng,  E->dact,
+  void* bufs[] = {E->qp,       E->qv,      E->pa,        E->steps,   E->rng,
                   E->zero_act, E->bench_r, E->bench_d,   E->ncon_hist, E->Wp,  E->dout,
-                  E->qflags,   E->qctr,    E->qerr,      E->qacc_e,  E->qacc_vx, E->tflags, E->tcount, E->tperm,
+                  E->qflags,   E->qctr,    E->qacc_e,  E->qacc_vx, E->tflags, E->tcount, E->tperm,
                   E->cflag,    E->Wt,      E->scr};
   for (void* b : bufs)
     if (b) HIPCHECK(hipFree(b));
   if (E->h_act) HIPCHECK(hipHostFree(E->h_act));
   if (E->h_out) HIPCHECK(hipHostFree(E->h_out));
-  if (E->h_qerr) HIPCHECK(hipHostFree(E->h_qerr));
+  if (E->qerr) HIPCHECK(hipHostFree(E->qerr));
   for (auto e : E->ev_phys) (void)hipEventDestroy(e);
   for (hipEvent_t e : E->step_ev) (void)hipEventDestroy(e);
   for (auto e : E->ev_pol) (void)hipEventDestroy(e);
   delete E;
 }
 
+// Whether the host-step path's kernels write their outputs straight into pinned host memory: batches that
+// fit the chip at once, whose step is a matter of tens of microseconds of copies and synchronisations
+// (us per step, through device memory and directly: 1 world 149, 122; 1024 282, 181; 4096 330, 269). Of
+// larger outputs the host copies one part while the next is transferred (8192 worlds 479; directly 513).
+static bool direct_outputs(const EnvState* E) { return E->N <= 2 * E->waves; }
+
+// The observations, and with rew the rewards and done flags, from the device's [obs | reward | done] to
+// the caller's arrays, through the pinned staging in chunks of worlds: the host copy of one chunk overlaps
+// the transfer of the next. Blocks.
+static void copy_outputs(EnvState* E, float* obs, float* rew, float* done) {
+  const size_t N = E->N, per = (N + kStepChunks - 1) / kStepChunks;
+  auto chunk = [&](int c, size_t& w0) { w0 = std::min(N, c * per); return std::min(N, w0 + per) - w0; };
+  for (int c = 0; c < kStepChunks; ++c) {
+    size_t w0;
+    if (const size_t n = chunk(c, w0))
+      HIPCHECK(hipMemcpyAsync(E->h_out + w0 * kObs, E->dout + w0 * kObs, n * kObs * 4, hipMemcpyDeviceToHost, 0));
+    HIPCHECK(hipEventRecord(E->step_ev[c], 0));
+  }
+  if (rew)
+    HIPCHECK(hipMemcpyAsync(E->h_out + N * kObs, E->dout + N * kObs, N * 2 * 4, hipMemcpyDeviceToHost, 0));
+  HIPCHECK(hipEventRecord(E->step_ev[kStepChunks], 0));
+  for (int c = 0; c < kStepChunks; ++c) {
+    HIPCHECK(hipEventSynchronize(E->step_ev[c]));
+    size_t w0;
+    if (const size_t n = chunk(c, w0)) std::memcpy(obs + w0 * kObs, E->h_out + w0 * kObs, n * kObs * 4);
+  }
+  HIPCHECK(hipEventSynchronize(E->step_ev[kStepChunks]));
+  if (rew) {
+    std::memcpy(rew, E->h_out + N * kObs, N * 4);
+    std::memcpy(done, E->h_out + N * (kObs + 1), N * 4);
+  }
+}
+
 void g1_env_reset(void* h, float* obs_out) {
   EnvState* E = (EnvState*)h;
-  poll_queue_error(E);
+  check_queue(E);
   const int N = E->N;
+  const bool direct = direct_outputs(E);
   hipLaunchKernelGGL(k_reset, dim3((N + 255) / 256), dim3(256), 0, 0, E->qp, E->qv, E->pa, E->steps, E->rng, N, 0.02f,
                      (const float*)nullptr, E->seed);
   HIPCHECK(hipGetLastError());
   hipLaunchKernelGGL(k_obs, dim3((unsigned)(((long)N * kObs + 255) / 256)), dim3(256), 0, 0, E->qp, E->qv, E->pa, N,
-                     E->dout);
+                     direct ? E->h_out : E->dout);
   HIPCHECK(hipGetLastError());
-  HIPCHECK(hipMemcpyAsync(E->h_out, E->dout, (size_t)N * kObs * 4, hipMemcpyDeviceToHost, 0));
+  if (!direct) {
+    copy_outputs(E, obs_out, nullptr, nullptr);
+    return;
+  }
   HIPCHECK(hipStreamSynchronize(0));
   std::memcpy(obs_out, E->h_out, (size_t)N * kObs * 4);
 }
 
-// Host-step path (reference: src/g1_env.cu:245-268,431-441): actions staged through pinned memory,
-// one launch that also writes the observation, one device-to-host copy of [obs | reward | done].
+// Host-step path (reference: src/g1_env.cu:245-268,431-441): one launch that reads the actions from pinned
+// host memory and writes [obs | reward | done].
 void g1_env_step(void* h, const float* act, float* obs, float* rew, float* done) {
   EnvState* E = (EnvState*)h;
-  poll_queue_error(E);
-  const int N = E->N;
-  // The caller's arrays are pageable: they pass through the pinned staging in chunks of worlds,
-  // so the host copy of one chunk overlaps the DMA of another.
-  const size_t per = ((size_t)N + kStepChunks - 1) / kStepChunks;
-  for (int c = 0; c < kStepChunks; ++c) {
-    const size_t w0 = c * per, w1 = w0 + per < (size_t)N ? w0 + per : (size_t)N;
-    if (w0 >= w1) break;
-    std::memcpy(E->h_act + w0 * kAct, act + w0 * kAct, (w1 - w0) * kAct * 4);
-    HIPCHECK(hipMemcpyAsync(E->dact + w0 * kAct, E->h_act + w0 * kAct, (w1 - w0) * kAct * 4, hipMemcpyHostToDevice, 0));
-  }
+  check_queue(E);
+  const size_t N = E->N;
+  const bool direct = direct_outputs(E);
+  std::memcpy(E->h_act, act, N * kAct * 4);
   PhysArgs pa = phys_args(E);
-  pa.act = E->dact; pa.t0 = 0; pa.astep = 0; pa.rstep = 0;
-  pa.obs = E->dout; pa.R = E->dout + (size_t)N * kObs; pa.D = E->dout + (size_t)N * (kObs + 1);
+  pa.act = E->h_act; pa.t0 = 0; pa.astep = 0; pa.rstep = 0;
+  pa.obs = direct ? E->h_out : E->dout;
+  pa.R = pa.obs + N * kObs; pa.D = pa.obs + N * (kObs + 1);
   launch_physics(E, pa);
-  for (int c = 0; c < kStepChunks; ++c) {
-    const size_t w0 = c * per, w1 = w0 + per < (size_t)N ? w0 + per : (size_t)N;
-    if (w0 < w1)
-      HIPCHECK(hipMemcpyAsync(E->h_out + w0 * kObs, E->dout + w0 * kObs, (w1 - w0) * kObs * 4, hipMemcpyDeviceToHost, 0));
-    HIPCHECK(hipEventRecord(E->step_ev[c], 0));
+  if (direct) {
+    HIPCHECK(hipStreamSynchronize(0));
+    std::memcpy(obs, E->h_out, N * kObs * 4);
+    std::memcpy(rew, E->h_out + N * kObs, N * 4);
+    std::memcpy(done, E->h_out + N * (kObs + 1), N * 4);
+  } else {
+    copy_outputs(E, obs, rew, done);
   }
-  HIPCHECK(hipMemcpyAsync(E->h_out + (size_t)N * kObs, E->dout + (size_t)N * kObs, (size_t)N * 2 * 4,
-                          hipMemcpyDeviceToHost, 0));
-  HIPCHECK(hipMemcpyAsync(E->h_out + (size_t)N * (kObs + 2), E->qerr, sizeof(int), hipMemcpyDeviceToHost, 0));
-  HIPCHECK(hipEventRecord(E->step_ev[kStepChunks], 0));
-  for (int c = 0; c < kStepChunks; ++c) {
-    HIPCHECK(hipEventSynchronize(E->step_ev[c]));
-    const size_t w0 = c * per, w1 = w0 + per < (size_t)N ? w0 + per : (size_t)N;
-    if (w0 < w1) std::memcpy(obs + w0 * kObs, E->h_out + w0 * kObs, (w1 - w0) * kObs * 4);
-  }
-  HIPCHECK(hipEventSynchronize(E->step_ev[kStepChunks]));
-  int err;
-  std::memcpy(&err, E->h_out + (size_t)N * (kObs + 2), sizeof(int));
-  check_queue_error(err);
-  std::memcpy(rew, E->h_out + (size_t)N * kObs, (size_t)N * 4);
-  std::memcpy(done, E->h_out + (size_t)N * (kObs + 1), (size_t)N * 4);
+  check_queue(E);
 }
 
 void g1_rollout(void* h, int H, const float* W, const float* mean, const float* var, float* O, float* A, float* LP,
@@ -1173,7 +1182,7 @@ int g1_rollout_noalloc(void* h, int H, const float* W, const float* mean, const 
 
 void g1_env_bench_phys(void* h, int K) {
   EnvState* E = (EnvState*)h;
-  poll_queue_error(E);
+  check_queue(E);
   if (K <= 0) return;   // no control step (the reference's loop runs zero times)
   PhysArgs pa = phys_args(E);
   pa.K = K; pa.act = E->zero_act; pa.t0 = 0; pa.astep = 0; pa.rstep = 0; pa.R = E->bench_r; pa.D = E->bench_d;
@@ -1222,7 +1231,7 @@ void g1_occupancy_report(void) {
 // ---- additive exports (no counterpart in the reference ABI) --------------------------------
 void g1_env_set_state(void* h, const float* qp, const float* qv, const float* pa, const int* steps) {
   EnvState* E = (EnvState*)h;
-  poll_queue_error(E);
+  check_queue(E);
   const size_t N = E->N;
   HIPCHECK(hipMemcpy(E->qp, qp, N * kNQ * 4, hipMemcpyHostToDevice));
   HIPCHECK(hipMemcpy(E->qv, qv, N * kNV * 4, hipMemcpyHostToDevice));
@@ -1304,9 +1313,7 @@ void g1_env_profile_read(void* h, double* out4) {
 int g1_env_check(void* h) {
   EnvState* E = (EnvState*)h;
   HIPCHECK(hipDeviceSynchronize());
-  int err = 0;
-  HIPCHECK(hipMemcpy(&err, E->qerr, sizeof(int), hipMemcpyDeviceToHost));
-  return err;
+  return *(volatile int*)E->qerr;
 }
 
 int g1_env_set_fused(void* h, int on) {

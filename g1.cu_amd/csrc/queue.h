@@ -30,7 +30,7 @@ struct PhysArgs {
   int qpar;                        //   clears row qpar ^ 1 for the next launch
   float* acc;                      // [N][32] per-lane energy sums of a control step split over items
   float* vxs;                      // [N] base x-velocity sum of a control step split over items
-  int* qerr;                       // 1: a dependency wait exceeded kSpinLimit polls; 2: a wave of
+  int* qerr;                       // (pinned host memory) 1: a dependency wait exceeded kSpinLimit polls; 2: a wave of
                                    //   queue q ran outside XCD q while xlocal is set
   int xlocal;                      // queue q's waves all run on XCD q (checked at env creation)
   int nch;                         // work items (substep chunks) per pair and control step:

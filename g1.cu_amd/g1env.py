@@ -111,7 +111,6 @@ class Env:
     def __init__(self, n_worlds, substeps=10, pgs_iters=8, seed=0):
         self.N, self.S, self.pgs, self.seed = int(n_worlds), int(substeps), int(pgs_iters), int(seed)
         self.h = lib.g1_env_create(self.N, self.S, self.pgs, self.seed)
-        self._io = None
 
     # ---- lifetime
     def close(self):
@@ -126,22 +125,17 @@ class Env:
         self.close()
 
     # ---- host-step path
-    def _buffers(self):
-        if self._io is None:
-            self._io = (np.empty((self.N, OBS_DIM), np.float32), np.empty(self.N, np.float32),
-                        np.empty(self.N, np.float32))
-        return self._io
-
     def reset(self):
-        obs, _, _ = self._buffers()
+        obs = np.empty((self.N, OBS_DIM), np.float32)
         lib.g1_env_reset(self.h, host_ptr(obs))
-        return obs.copy()
+        return obs
 
     def step(self, actions):
-        obs, rew, done = self._buffers()
+        obs, rew, done = (np.empty((self.N, OBS_DIM), np.float32), np.empty(self.N, np.float32),
+                          np.empty(self.N, np.float32))
         act = np.ascontiguousarray(actions, np.float32).reshape(self.N, ACT_DIM)
         lib.g1_env_step(self.h, host_ptr(act), host_ptr(obs), host_ptr(rew), host_ptr(done))
-        return obs.copy(), rew.copy(), done.copy()
+        return obs, rew, done
 
     def qpos_all(self):
         out = np.empty((self.N, NQ), np.float32)

@@ -75,8 +75,8 @@ void g1_rollout_ex(void* h, int H, const float* W, const float* mean, const floa
  * All calls on one GPU share the array; the library orders its launches on the null stream, so
  * successive calls do not overlap, and callers must not run two of them concurrently on other
  * streams. Asynchronous, like g1_rollout; no profiling events are recorded. Not for HIP graph
- * capture: its launches and its closing error-word copy go to the null stream, and it reads the
- * previous rollout's error word from host memory on entry. */
+ * capture: its launches go to the null stream, and it reads the work queue's error word from host
+ * memory on entry. */
 int g1_rollout_noalloc(void* h, int H, const float* W, const float* mean, const float* var, float* O, float* A,
                        float* LP, float* V, float* R, float* D, float* Vlast, const float* act_noise,
                        const float* reset_noise);
