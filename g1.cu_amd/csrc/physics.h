@@ -620,18 +620,13 @@ __device__ __forceinline__ void base_solve(const WorldLds& s, const float (&xb)[
 }
 
 // Ordering point between the phases of world_qacc, whose callers run it in workgroups of one wave
-// (k_physics, k_rollout, k_probe: 64 threads). A wave's LDS accesses are performed in program
-// order, so a wavefront-scope fence (the compiler keeps the accesses in order; no instruction) is
-// all a hand-over through LDS between its lanes needs; __syncthreads() adds an lgkmcnt(0) drain of
-// every outstanding LDS access at each phase boundary. The translation unit of k_rollout defines
-// G1_PHASE_FENCE and takes the fence: config 3 10.50 -> 10.43 ms; k_physics keeps the barrier
-// (with the default scheduler it was faster, 194.4 against 193.3 ms at config 4; with the ILP-first
-// one both measure the same).
-#ifdef G1_PHASE_FENCE
+// (k_physics, k_rollout, k_resident, k_probe: 64 threads). A wave's LDS accesses are performed in
+// program order, so a wavefront-scope fence (the compiler keeps the accesses in order; no instruction)
+// is all a hand-over through LDS between its lanes needs; __syncthreads() adds an lgkmcnt(0) drain of
+// every outstanding LDS access at each phase boundary: the training rollout 10.50 -> 10.43 ms when the
+// fence came in; k_physics and k_probe followed later (50 steps of 8192 standing worlds 19.00 -> 18.93
+// ms, a host step of 8192 485 -> 480 us, ten contact-free substeps 181.0 -> 179.9 us).
 __device__ __forceinline__ void wave_sync() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
-#else
-__device__ __forceinline__ void wave_sync() { __syncthreads(); }
-#endif
 
 // The chain layout's stores without a lane test (the factor, the force gather, the RNE staging): a
 // chain outside its depth range writes the row of body c_off + depth, which its owner must store

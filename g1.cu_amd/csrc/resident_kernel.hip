@@ -1,8 +1,7 @@
 // resident_kernel.hip -- k_resident: a whole rollout, or K control steps on given actions, with one or two
-// worlds per wave (resident.h). Its own translation unit for the wavefront-fence phase boundaries.
+// worlds per wave (resident.h).
 #include <hip/hip_runtime.h>
 
-#define G1_PHASE_FENCE   // world_qacc's phase boundaries as wavefront fences (see wave_sync)
 #include "resident.h"
 
 namespace g1k {

@@ -1,9 +1,8 @@
 // rollout_kernel.hip -- k_rollout, the whole g1_rollout in one persistent launch (the scheme and
-// its argument block are described in queue.h). Its own translation unit, so that it alone takes
-// the wavefront-fence phase boundaries (G1_PHASE_FENCE below).
+// its argument block are described in queue.h). Its own translation unit for its compiler flags
+// (build.py).
 #include <hip/hip_runtime.h>
 
-#define G1_PHASE_FENCE   // world_qacc's phase boundaries as wavefront fences (see wave_sync)
 #include "queue.h"
 
 namespace g1k {
