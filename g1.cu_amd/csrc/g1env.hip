@@ -763,26 +763,33 @@ static void chunk_schedule(PhysArgs& a, int pgrid, bool one_launch = false) {
   a.nchl = build(big ? 1 : 2, a.cstl);
 }
 
-// Worlds per wave of the resident form (k_resident), or 0 where the work queue runs the launch: one while
-// every wave can have a SIMD to itself (1024 worlds), two while all waves are resident at once (4096).
-// Measured, ms per 32 steps of the 256-256 policy with one world per wave, two, and the queue: 1024
-// worlds 3.38, 3.85, 5.42; 1536 3.86, 3.87, 5.48; 2048 3.99, 3.81, 5.51; 4096 -, 4.46, 6.02; past that
+// The form of a launch: worlds per wave and waves per world of k_resident, or worlds 0: the work queue. One
+// world on two waves while every wave can have a SIMD to itself (512 worlds), one per wave while that
+// holds for them (1024), two per wave while all waves are resident at once (4096). Measured, ms per
+// rollout of the 256-256 policy on two waves, with one world per wave, two, and the queue: 16 steps of 256
+// worlds 1.50, 1.63, 1.83, 2.55; 32 steps of 1024 -,
+// 3.38, 3.85, 5.42; 1536 -, 3.86, 3.87, 5.48; 2048 -, 3.99, 3.81, 5.51; 4096 -, -, 4.46, 6.02; past that
 // a second round of waves would start when the first ends, and the queue spreads the work evenly (8192
-// worlds 7.6). Control steps on given actions, us per 20 steps of standing robots: 64 worlds 3452, 3504,
-// 3599; 1024 3615, 3696, 3758; 2048 4162, 3604, 3723; 4096 -, 4176, 4224. An env set to the fenced hand-over keeps the queue, which that mode is about.
-static int resident_worlds(const EnvState* E) {
-  if (E->fences) return 0;
-  return E->N <= E->waves / 2 ? 1 : (E->N <= 2 * E->waves ? 2 : 0);
+// worlds 7.6). Control steps on given actions, us per 20 steps of standing robots with one, two and the
+// queue: 64 worlds 3452, 3504, 3599; 1024 3615, 3696, 3758; 2048 4162, 3604, 3723; 4096 -, 4176, 4224.
+// An env set to the fenced hand-over keeps the queue, which that mode is about.
+struct ResidentForm { int worlds, waves; };
+static ResidentForm resident_form(const EnvState* E) {
+  if (E->fences) return {0, 0};
+  if (E->N <= E->waves / 4) return {1, 2};
+  if (E->N <= E->waves / 2) return {1, 1};
+  return {E->N <= 2 * E->waves ? 2 : 0, 1};
 }
 
 // Enqueue one physics launch on the null stream; the queue state (flag base, counter row) advances
 // on the host in launch order, which is the stream's execution order.
 static void launch_physics(EnvState* E, PhysArgs& a) {
   if (a.K <= 0) fail("physics launch: K must be positive");
-  if (const int per_wave = resident_worlds(E)) {
+  const ResidentForm form = resident_form(E);
+  if (form.worlds) {
     ResidentArgs ra{};
     ra.ph = a;
-    launch_resident_kernel(ra, false, per_wave == 2);
+    launch_resident_kernel(ra, false, form.worlds, form.waves);
     HIPCHECK(hipGetLastError());
     return;
   }
@@ -814,7 +821,7 @@ static void check_queue(EnvState* E) { check_queue_error(*(volatile int*)E->qerr
 // The one-launch rollout runs policies of two hidden layers of at most 256 units each on the
 // register-resident tile (policy_tile, at 256-256 with zero padding) and every other accepted shape
 // (1..3 hidden layers of at most 512 units) on the wide tile (policy_tile_wide, activations staged
-// in global memory); small batches of either kind run resident waves (resident_worlds). The split form
+// in global memory); small batches of either kind run resident waves (resident_form). The split form
 // (policy and physics launches per control step) remains for g1_env_set_fused(h, 0) and for
 // g1_rollout_noalloc with a wide shape (the wide tile's activation buffers are allocated by the library).
 static bool narrow_shape(const PolicyShape& sh) {
@@ -854,7 +861,7 @@ static void pack_wide(EnvState* E, const float* W, const float* mean, const floa
 }
 
 // The whole rollout as one k_resident launch on the null stream; wp as in rollout_fused.
-static void rollout_resident(EnvState* E, int per_wave, int H, const float* W, const float* mean, const float* var,
+static void rollout_resident(EnvState* E, ResidentForm form, int H, const float* W, const float* mean, const float* var,
                              float* O, float* A, float* LP, float* V, float* R, float* D, float* Vlast,
                              const float* act_noise, const float* reset_noise, float* wp, long wp_cap) {
   const WideLayout wl = wide_layout(E->shape.nl, E->shape.hid, E->shape.act);
@@ -867,7 +874,7 @@ static void rollout_resident(EnvState* E, int per_wave, int H, const float* W, c
   ra.po = TileArgs{Wt, TileLayout{}, act_noise, O, A, LP, V, Vlast, H, 1, wl, nullptr};
   const bool prof = E->prof_on != 0 && !wp;
   if (prof) prof_mark(E->ev_phys, E->n_phys);
-  launch_resident_kernel(ra, true, per_wave == 2);
+  launch_resident_kernel(ra, true, form.worlds, form.waves);
   HIPCHECK(hipGetLastError());
   if (prof) prof_mark(E->ev_phys, E->n_phys);
 }
@@ -928,8 +935,9 @@ static void rollout_impl(EnvState* E, int H, const float* W, const float* mean, 
   check_queue(E);
   if (H < 0) H = 0;   // no control step; the bootstrap value is still computed (as the reference's k_rollout)
   if (E->fused && fused_shape(E->shape, wp != nullptr)) {
-    if (const int per_wave = resident_worlds(E)) {
-      rollout_resident(E, per_wave, H, W, mean, var, O, A, LP, V, R, D, Vlast, act_noise, reset_noise, wp, wp_cap);
+    const ResidentForm form = resident_form(E);
+    if (form.worlds) {
+      rollout_resident(E, form, H, W, mean, var, O, A, LP, V, R, D, Vlast, act_noise, reset_noise, wp, wp_cap);
       return;
     }
     rollout_fused(E, H, W, mean, var, O, A, LP, V, R, D, Vlast, act_noise, reset_noise, wp, wp_cap);
@@ -1213,8 +1221,9 @@ void g1_occupancy_report(void) {
   struct { const char* nm; const void* fn; int threads; size_t smem; } ks[] = {
       {"k_rollout", rollout_kernel_fn(false), kPhysThreads, 0},
       {"k_rollout (wide)", rollout_kernel_fn(true), kPhysThreads, 0},
-      {"k_resident (1)", resident_kernel_fn(false), kPhysThreads, 0},
-      {"k_resident (2)", resident_kernel_fn(true), kPhysThreads, 0},
+      {"k_resident (1/2)", resident_kernel_fn(1, 2), 2 * kPhysThreads, 0},
+      {"k_resident (1)", resident_kernel_fn(1, 1), kPhysThreads, 0},
+      {"k_resident (2)", resident_kernel_fn(2, 1), kPhysThreads, 0},
       {"k_physics", (const void*)k_physics, kPhysThreads, 0},
       {"k_policy", (const void*)k_policy, kPolicyThreads, policy_smem(PolicyShape{2, {256, 256, 0, 0}, 0})},
       {"k_probe", (const void*)k_probe, kPhysThreads, 0}};

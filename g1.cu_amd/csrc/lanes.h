@@ -11,7 +11,7 @@ namespace g1k {
 constexpr int kGroup = 32;
 
 __device__ __forceinline__ int group_lane() { return threadIdx.x & (kGroup - 1); }
-__device__ __forceinline__ int group_id() { return threadIdx.x >> 5; }
+__device__ __forceinline__ int group_id() { return (threadIdx.x >> 5) & 1; }   // half of the wave
 
 __device__ __forceinline__ float gshfl(float v, int src) { return __shfl(v, src, kGroup); }
 __device__ __forceinline__ int gshfl(int v, int src) { return __shfl(v, src, kGroup); }

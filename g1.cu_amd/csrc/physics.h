@@ -651,12 +651,31 @@ constexpr bool hinge_armature_uniform() {
   return true;
 }
 
+// The LDS of a world on two waves beside WorldLds: the RNE staging and the bodies' forces, which wave 1
+// keeps while wave 0 fills the places they take otherwise, and the pelvis' articulated bias.
+struct DuoLds {
+  alignas(16) float VA[kNBody * 20];
+  alignas(16) float Fo[kNBody * 6];
+  alignas(16) float pA[6];
+};
+__device__ __forceinline__ void duo_sync() { __syncthreads(); }
+
 // ================================================================ substep: qacc of one world
 // Inputs: lane state, PD torque of the lane's hinge dof (jtau). Output: qacc of the lane's dofs
 // (every lane: the 6 base dofs into bqacc[]; hinge lanes: jqacc). Returns this world's contact count.
-// Must be called by all 64 lanes of the block in uniform control flow.
+// Must be called by all 64 lanes of the wave in uniform control flow.
+//
+// kDuo: the world on two waves of one block (k_resident's small batches, where SIMDs stand idle). Both
+// call it with the same state and form the frames; then wave 0 (role 0) runs the inertias, the factor
+// and the free joint's Cholesky while wave 1 runs the bias forces, then the smooth solve's leaf -> root
+// sweep (fused into the factor otherwise); wave 0 forms the contact rows meanwhile and finishes the
+// solves. The operations on every value are those of one wave, so the results are too. Hand-overs between the waves
+// are block barriers, the same four on either wave (duo_sync #1 .. #4); what the waves would overwrite
+// of each other lies in `duo` (DuoLds) instead.
+template <bool kDuo = false>
 __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState& st, float jtau,
-                                          const SolveParams& P, float (&bqacc)[6], float& jqacc) {
+                                          const SolveParams& P, float (&bqacc)[6], float& jqacc, int role = 0,
+                                          DuoLds* duo = nullptr) {
   // The lane index goes through an opaque asm on every call so the per-lane model constants are
   // re-read from the (cached) tables each substep instead of being hoisted out of the caller's
   // substep loop, where they would occupy ~150 registers for the whole kernel.
@@ -779,7 +798,7 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
     const bool hit = (l < kNFoot) && (pen < 0.f);
     const unsigned mask = group_ballot8(hit);
     ncon = __popc(mask);
-    if (hit) {
+    if (hit && (!kDuo || role == 0)) {
       const int idx = __popc(mask & ((1u << l) - 1u));
       s.con[idx][0] = c.x; s.con[idx][1] = c.y; s.con[idx][2] = pen * 0.5f; s.con[idx][3] = pen;
       s.con_w0[idx] = foot_w0;
@@ -794,7 +813,7 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
   V3 sw{0.f, 0.f, 0.f}, sv{0.f, 0.f, 0.f};   // hinge axis (angular; linear)
   // the pelvis rotation on every lane (the free joint's right-hand side and base solve use it)
   const M3 R1 = quat2mat(qpel);
-  if (L.hinge) {
+  if (L.hinge && (!kDuo || role == 0)) {
     sw = qrot(xq, L.axis);
     sv = cross(vsub(xp, p), sw);
     const int d = L.b + 4;
@@ -803,7 +822,7 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
     s.u.fac.S[d][6] = L.bdt;   // the row's padding carries the factor's dt kd (column 7: x_b)
     s.qvel[d] = st.jqd;
   }
-  if (base) {
+  if (base && (!kDuo || role == 0)) {
     // only the rotations' angular parts (R1 columns) are stored: every use of the free joint's
     // subspace takes its structure from sbase_dot / sbase_col
 #pragma unroll
@@ -877,9 +896,11 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
   // more): every level's slot sits at an immediate offset from the lane's base, and the body stride
   // of 20 words puts the four chains' rows of a level on different LDS banks
   constexpr int kVA = 20;
-  float* const V6 = &s.Mm[0][0];
+  float* const V6 = kDuo ? duo->VA : &s.Mm[0][0];
   float* const A6 = V6 + kVA / 2;
   static_assert(kCols * kMmStride >= kNBody * kVA && kVA / 2 >= 8, "RNE staging fits the solve-output region");
+  if (kDuo) duo_sync();   // #1: the motion axes, velocities and contact points of wave 0 in LDS
+  if (!kDuo || role == 1) {
   if (base) {
     V6[kVA + 0] = vw.x; V6[kVA + 1] = vw.y; V6[kVA + 2] = vw.z; V6[kVA + 3] = vv.x; V6[kVA + 4] = vv.y; V6[kVA + 5] = vv.z;
     A6[kVA + 0] = aw.x; A6[kVA + 1] = aw.y; A6[kVA + 2] = aw.z; A6[kVA + 3] = av.x; A6[kVA + 4] = av.y; A6[kVA + 5] = av.z;
@@ -967,6 +988,7 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
     vw = {v6[0], v6[1], v6[2]}; vv = {v6[3], v6[4], v6[5]};
     aw = {a6[0], a6[1], a6[2]}; av = {a6[3], a6[4], a6[5]};
   }
+  }
 
   // ---------------- body forces f = I a + v x* (I v) (reference: src/aba_bias.cuh:103-111,
   // inertia application src/dynamics.cuh:126-139)
@@ -983,7 +1005,7 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
     fv = {fmaf_(m, xv.x, -m * cs.x), fmaf_(m, xv.y, -m * cs.y), fmaf_(m, xv.z, -m * cs.z)};
   };
   V3 Fw{0.f, 0.f, 0.f}, Fv{0.f, 0.f, 0.f};
-  if (L.body) {
+  if (L.body && (!kDuo || role == 1)) {
     V3 Iaw, Iav, Ivw, Ivv;
     apply_I(aw, av, Iaw, Iav);
     apply_I(vw, vv, Ivw, Ivv);
@@ -1000,12 +1022,12 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
   // The bodies' own forces go to the hinge-factor column rows (U), which the factor overwrites only
   // for the hinge bodies 2..30: the pelvis' subtree force (row 1) is read after the factor.
   static_assert(sizeof(float) * kNBody * kRow >= sizeof(float) * kNBody * 6, "force staging fits U");
-  float* const Fo = &s.u.fac.U[0][0];     // [kNBody][6] each body's own RNE force (w, v)
-  if (L.body) {
+  float* const Fo = kDuo ? duo->Fo : &s.u.fac.U[0][0];     // [kNBody][6] each body's own RNE force (w, v)
+  if (L.body && (!kDuo || role == 1)) {
     Fo[6 * L.b + 0] = Fw.x; Fo[6 * L.b + 1] = Fw.y; Fo[6 * L.b + 2] = Fw.z;
     Fo[6 * L.b + 3] = Fv.x; Fo[6 * L.b + 4] = Fv.y; Fo[6 * L.b + 5] = Fv.z;
   }
-  if (L.body) {
+  if (L.body && (!kDuo || role == 0)) {
     const float c2 = dot3(cc, cc);
     float A[9];
 #pragma unroll
@@ -1039,7 +1061,7 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
   // closes the sweep. The chain is one addition per level with no exchange inside the chain, and
   // each hinge lane then takes its own body's F from LDS for S_b.F_b (the lane-per-body form's
   // order), so the factor's sweep only reads x_b.
-  {
+  if (!kDuo || role == 1) {
     float* const pF = Fo + 6 * c_off + rowc;
     // every level's own force read before the sweep (each level reads its own slot once, before
     // it stores it): the reads go out together instead of one LDS round trip per level, which the
@@ -1071,7 +1093,7 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
     if (l < 6) Fo[6 + l] = F1;
   }
   wave_sync();   // every subtree force in LDS
-  if (L.hinge) {
+  if (L.hinge && (!kDuo || role == 1)) {
     const float* const Fb = Fo + 6 * L.b;
     const float* const Sb = s.u.fac.S[L.b + 4];   // (w, v) of the hinge axis, as stored above
     float bias = Sb[0] * Fb[0];
@@ -1147,7 +1169,7 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
     float D = dot6(Sd, Ub) + arm;
     if (P.damped) D += bdt;
     const float invD = rcp_rn(D);
-    const float u = xb_ - dot6(Sd, pA);
+    const float u = kDuo ? 0.f : xb_ - dot6(Sd, pA);   // kDuo: wave 1's sweep, which stores it after #2
     const float ud = u * invD;
 #pragma unroll
     for (int j = 0; j < 6; ++j) {
@@ -1171,6 +1193,7 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
   // go ahead of the other wave's wider phases. Same-box A/B, ms per rollout: config 3 12.69 ->
   // 12.54, config 4 232.5 -> 230.1 (priority raised for FK or RNE as well was slower, for PGS
   // alone 12.64).
+  if (!kDuo || role == 0) {
   __builtin_amdgcn_s_setprio(1);
   prefetch(kMaxDepth);
   prefetch(kMaxDepth - 1);
@@ -1188,6 +1211,112 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
   }
 #pragma unroll
   for (int cd = kTorsoDepth - 1; cd >= 2; --cd) level(cd, false, none, none);
+  }
+  // ---------------- PASS 1: basis rows, R, aref (reference: src/env_qacc.cuh:67-136)
+  auto pass1 = [&]() {
+  const float mu = P.mu;
+  static_assert(kContactDofs == 12 && 2 * kContactDofs <= kGroup, "two contacts' rows per pass");
+  if (ncon_max > 0) {
+    // the basis rows, lane-parallel: in pass ps lane l < 24 forms the three entries of contact
+    // 2 ps + l / 12 on its ancestor dof k = l mod 12, walked foot -> root: leg hinges (foot first),
+    // then the free base 0..5. Point Jacobian column w x r + lv; on the free base the structural
+    // zeros of S_base are skipped (see sbase_dot): translation a gives e_a, rotation a gives w x r.
+    const int k = l % kContactDofs;
+#pragma unroll
+    for (int ps = 0; ps < (kNFoot + 1) / 2; ++ps) {
+      if (2 * ps >= ncon_max) break;
+      const int ci = 2 * ps + l / kContactDofs;
+      const bool on = l < 2 * kContactDofs && ci < ncon;
+      const int c = on ? ci : 0;
+      const int a = (k < 6) ? (s.con_leg[c] ? 12 : 6) + 5 - k : k - 6;
+      const V3 r = vsub(V3{s.con[c][0], s.con[c][1], s.con[c][2]}, p);
+      const float* Sa = s.u.fac.S[a];   // (base translation rows: never stored, unused)
+      const V3 cr = cross(V3{Sa[0], Sa[1], Sa[2]}, r);
+      const V3 leg = vadd(cr, V3{Sa[3], Sa[4], Sa[5]});
+      const bool trans = k >= 6 && a < 3;
+      const V3 jc{k < 6 ? leg.x : (trans ? (a == 0 ? 1.f : 0.f) : cr.x),
+                  k < 6 ? leg.y : (trans ? (a == 1 ? 1.f : 0.f) : cr.y),
+                  k < 6 ? leg.z : (trans ? (a == 2 ? 1.f : 0.f) : cr.z)};
+      if (on) { s.Eb[c][0][k] = jc.z; s.Eb[c][1][k] = mu * jc.y; s.Eb[c][2][k] = -mu * jc.x; }
+    }
+  }
+  wave_sync();   // the basis rows in LDS
+  if (ncon_max > 0 && l < ncon) {
+    const int c = l;
+    const int legbase = s.con_leg[c] ? 12 : 6;
+    // the reference velocities of the four pyramid rows: sum_k e_a[k] qd[k] in dof order
+    float v0 = 0.f, v1 = 0.f, v2 = 0.f;
+#pragma unroll
+    for (int k = 0; k < kContactDofs; ++k) {
+      const float qd = s.qvel[(k < 6) ? legbase + 5 - k : k - 6];
+      v0 = fmaf_(s.Eb[c][0][k], qd, v0); v1 = fmaf_(s.Eb[c][1][k], qd, v1); v2 = fmaf_(s.Eb[c][2][k], qd, v2);
+    }
+    const float dmax = MF::foot_solimp[1], tc = MF::foot_solref[0], dr = MF::foot_solref[1];
+    const float bcoef = 2.f / (dmax * tc);
+    const float kcoef = 1.f / (dmax * dmax * tc * tc * dr * dr);
+    const float pyr = (1.f + mu * mu) * (2.f * mu * mu / MF::foot_impratio);
+    const float pen = s.con[c][3], imp = foot_impedance(pen);
+    s.Rc[c] = div_rn(s.con_w0[c] * pyr * (1.f - imp), imp, rcp_rn(imp));
+    const float kip = kcoef * imp * pen;
+    s.aref[4 * c + 0] = -bcoef * (v0 + v1) - kip;
+    s.aref[4 * c + 1] = -bcoef * (v0 - v1) - kip;
+    s.aref[4 * c + 2] = -bcoef * (v0 + v2) - kip;
+    s.aref[4 * c + 3] = -bcoef * (v0 - v2) - kip;
+  }
+  wave_sync();
+  };
+
+  if (kDuo && role == 1) {
+    // The smooth solve's leaf -> root sweep on its own (see `level`, which fuses it otherwise): every lane
+    // of a chain carries the whole articulated bias force; operands read a level ahead (all of them
+    // before the sweep: no faster, and past two waves per SIMD's registers).
+    const float* const pU = &s.u.fac.U[c_off][0];
+    float Sa[8], Ua[8], Sb[8], Ub[8];
+    auto ld = [&](int cd, float (&S8)[8], float (&U8)[8]) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) { S8[j] = pSc[kRow * cd + j]; U8[j] = pU[kRow * cd + j]; }
+    };
+    auto sweep = [&](int cd, const float (&S8)[8], const float (&U8)[8]) {
+      const bool act = cd >= c_lo && cd <= c_hi, leaf = cd == c_hi;
+      float pA[6], Sd[6];
+#pragma unroll
+      for (int j = 0; j < 6; ++j) {
+        Sd[j] = S8[j];
+        float g = cs[j];
+        if (cd == kTorsoDepth) {   // the right arm's bias force joins the torso first (chain 3 -> 2)
+          const float gc = from_next_chain(cs[j]);
+          g = grp == 2 ? gc + cs[j] : cs[j];
+        }
+        pA[j] = leaf ? 0.f : g;
+      }
+      const float u = S8[7] - dot6(Sd, pA);
+      const float ud = u * U8[kInvD];
+#pragma unroll
+      for (int j = 0; j < 6; ++j) cs[j] = fmaf_(U8[j], ud, pA[j]);
+      if (act && crow == 0) s.u.fac.U[c_off + cd][kUs] = u;
+    };
+    duo_sync();   // #2: the factor (wave 0); x_b and the pelvis' subtree force (wave 1)
+    ld(kMaxDepth, Sa, Ua);
+#pragma unroll
+    for (int cd = kMaxDepth; cd >= 2; --cd) {
+      const bool odd = (kMaxDepth - cd) & 1;
+      if (cd > 2) ld(cd - 1, odd ? Sa : Sb, odd ? Ua : Ub);
+      sweep(cd, odd ? Sb : Sa, odd ? Ub : Ua);
+    }
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+      const float c14 = from_upper_row(cs[j]), c8 = from_next_chain(cs[j]);
+      const float v = (c14 + c8) + cs[j];
+      if (l == 0) duo->pA[j] = v;
+    }
+    duo_sync();   // #3: the biases u and pA_1 (wave 1)
+    duo_sync();   // #4: qacc (wave 0)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) bqacc[k] = s.qacc[k];
+    jqacc = L.hinge ? s.qacc[L.b + 4] : 0.f;
+    return ncon;
+  }
+  if (kDuo) duo_sync();   // #2
   // pelvis: I^A_1 = I6_1 + D_14 + D_8 + D_2 and pA_1 = cs_14 + cs_8 + cs_2 (descending children),
   // row r on lane r of chain 0, which all hold pA_1
   float pAs[6], I1[6];
@@ -1251,7 +1380,7 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
   // pA_1 from lane 1 (chain 0's lanes hold it) to every lane for the smooth base solve (waves
   // without contacts), while D is built and read
   float pA1[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if (ncon_max == 0) {
+  if (!kDuo && ncon_max == 0) {
 #pragma unroll
     for (int k = 0; k < 6; ++k) pA1[k] = gshfl(pAs[k], 1);
   }
@@ -1283,6 +1412,12 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
           Dm[i * 6 + j] = div_rn(a, Dm[j * 6 + j], Dinv[j]);
         }
       }
+    if (kDuo) {
+      pass1();      // (independent of the smooth solve: while wave 1 ends its sweep)
+      duo_sync();   // #3
+#pragma unroll
+      for (int k = 0; k < 6; ++k) pAs[k] = pA1[k] = duo->pA[k];
+    }
     // With contacts the smooth solve's base and root -> leaf parts run as column 0 of the contact
     // solves below (lane 0, the same operations in the same order), which read the factor from LDS
     // (the lower triangle); without, here and in the level-synchronous sweep.
@@ -1364,62 +1499,12 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
       const float q = (usc - dot6(Uc, a)) * iDc;
 #pragma unroll
       for (int k = 0; k < 6; ++k) a[k] = fmaf_(Sc[k], q, a[k]);
-      if (r >= c_lo && r <= c_hi && crow == 0) s.Mm[0][chain_body(r) + 4] = q;
+      if (r >= c_lo && r <= c_hi && crow == 0) (kDuo ? s.qacc : s.Mm[0])[chain_body(r) + 4] = q;
     }
   }
 
   __builtin_amdgcn_s_setprio(3);   // the contact pipeline (see the factor above)
-  // ---------------- PASS 1: basis rows, R, aref (reference: src/env_qacc.cuh:67-136)
-  const float mu = P.mu;
-  static_assert(kContactDofs == 12 && 2 * kContactDofs <= kGroup, "two contacts' rows per pass");
-  if (ncon_max > 0) {
-    // the basis rows, lane-parallel: in pass ps lane l < 24 forms the three entries of contact
-    // 2 ps + l / 12 on its ancestor dof k = l mod 12, walked foot -> root: leg hinges (foot first),
-    // then the free base 0..5. Point Jacobian column w x r + lv; on the free base the structural
-    // zeros of S_base are skipped (see sbase_dot): translation a gives e_a, rotation a gives w x r.
-    const int k = l % kContactDofs;
-#pragma unroll
-    for (int ps = 0; ps < (kNFoot + 1) / 2; ++ps) {
-      if (2 * ps >= ncon_max) break;
-      const int ci = 2 * ps + l / kContactDofs;
-      const bool on = l < 2 * kContactDofs && ci < ncon;
-      const int c = on ? ci : 0;
-      const int a = (k < 6) ? (s.con_leg[c] ? 12 : 6) + 5 - k : k - 6;
-      const V3 r = vsub(V3{s.con[c][0], s.con[c][1], s.con[c][2]}, p);
-      const float* Sa = s.u.fac.S[a];   // (base translation rows: never stored, unused)
-      const V3 cr = cross(V3{Sa[0], Sa[1], Sa[2]}, r);
-      const V3 leg = vadd(cr, V3{Sa[3], Sa[4], Sa[5]});
-      const bool trans = k >= 6 && a < 3;
-      const V3 jc{k < 6 ? leg.x : (trans ? (a == 0 ? 1.f : 0.f) : cr.x),
-                  k < 6 ? leg.y : (trans ? (a == 1 ? 1.f : 0.f) : cr.y),
-                  k < 6 ? leg.z : (trans ? (a == 2 ? 1.f : 0.f) : cr.z)};
-      if (on) { s.Eb[c][0][k] = jc.z; s.Eb[c][1][k] = mu * jc.y; s.Eb[c][2][k] = -mu * jc.x; }
-    }
-  }
-  wave_sync();   // the basis rows in LDS
-  if (ncon_max > 0 && l < ncon) {
-    const int c = l;
-    const int legbase = s.con_leg[c] ? 12 : 6;
-    // the reference velocities of the four pyramid rows: sum_k e_a[k] qd[k] in dof order
-    float v0 = 0.f, v1 = 0.f, v2 = 0.f;
-#pragma unroll
-    for (int k = 0; k < kContactDofs; ++k) {
-      const float qd = s.qvel[(k < 6) ? legbase + 5 - k : k - 6];
-      v0 = fmaf_(s.Eb[c][0][k], qd, v0); v1 = fmaf_(s.Eb[c][1][k], qd, v1); v2 = fmaf_(s.Eb[c][2][k], qd, v2);
-    }
-    const float dmax = MF::foot_solimp[1], tc = MF::foot_solref[0], dr = MF::foot_solref[1];
-    const float bcoef = 2.f / (dmax * tc);
-    const float kcoef = 1.f / (dmax * dmax * tc * tc * dr * dr);
-    const float pyr = (1.f + mu * mu) * (2.f * mu * mu / MF::foot_impratio);
-    const float pen = s.con[c][3], imp = foot_impedance(pen);
-    s.Rc[c] = div_rn(s.con_w0[c] * pyr * (1.f - imp), imp, rcp_rn(imp));
-    const float kip = kcoef * imp * pen;
-    s.aref[4 * c + 0] = -bcoef * (v0 + v1) - kip;
-    s.aref[4 * c + 1] = -bcoef * (v0 - v1) - kip;
-    s.aref[4 * c + 2] = -bcoef * (v0 + v2) - kip;
-    s.aref[4 * c + 3] = -bcoef * (v0 - v2) - kip;
-  }
-  wave_sync();
+  if (!kDuo) pass1();   // (kDuo: run above)
 
   // ---------------- PASS 2: M^-1 solves, lane j = basis column j (reference: src/aba_factor.cuh:121-165,
   // src/env_qacc.cuh:137-152). Lane 0 finishes column 0, the smooth solve: its leaf -> root part
@@ -1641,7 +1726,13 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
   if (ncon_max == 0) {
 #pragma unroll
     for (int k = 0; k < 6; ++k) bqacc[k] = qb[k];   // every lane: each integrates the free joint
-    jqacc = L.hinge ? s.Mm[0][L.b + 4] : 0.f;
+    if (kDuo) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k)
+        if (l == 0) s.qacc[k] = qb[k];
+      duo_sync();   // #4
+    }
+    jqacc = L.hinge ? (kDuo ? s.qacc : s.Mm[0])[L.b + 4] : 0.f;
     __builtin_amdgcn_s_setprio(0);
     wave_sync();
     return ncon;
@@ -1915,7 +2006,8 @@ __device__ __forceinline__ int world_qacc(int lane, WorldLds& s, const LaneState
     s.qacc[d1] = s1 + dq1;
     if (kGroup + l < kNV) s.qacc[d2] = s2 + dq2;
   }
-  wave_sync();
+  if (kDuo) duo_sync();   // #4
+  else wave_sync();
 #pragma unroll
   for (int k = 0; k < 6; ++k) bqacc[k] = s.qacc[k];   // every lane: each integrates the free joint
   jqacc = L.hinge ? s.qacc[L.b + 4] : 0.f;

@@ -103,9 +103,11 @@ __device__ __forceinline__ float pd_target(const LaneModel& L, float act) {
 // Substeps [s0, s1) of a control step of the lane's world: PD torques, world_qacc, Euler (reference:
 // src/g1_env.cu:141-163). Adds to the step's energy and base-velocity sums; returns the contacts at
 // the last substep. hcnt: lane q < 9 counts the world's substeps with q contacts.
+// role, duo: the wave's part of a world on two waves (world_qacc).
+template <bool kDuo = false>
 __device__ __forceinline__ int run_substeps(const SolveParams& P, WorldLds& s, const LaneModel& L, int l, bool wvalid,
                                             float target, int s0, int s1, LaneState& st, float& energy, float& vx_sum,
-                                            unsigned& hcnt) {
+                                            unsigned& hcnt, int role = 0, DuoLds* duo = nullptr) {
   int nc_last = 0;
 #pragma unroll 1
   for (int sub = s0; sub < s1; ++sub) {
@@ -118,7 +120,7 @@ __device__ __forceinline__ int run_substeps(const SolveParams& P, WorldLds& s, c
       energy += fabsf(pdt * st.jqd);
     }
     float bqacc[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, jqacc = 0.f;
-    const int nc = world_qacc(l, s, st, jtau, P, bqacc, jqacc);
+    const int nc = world_qacc<kDuo>(l, s, st, jtau, P, bqacc, jqacc, role, duo);
     hcnt += (l == nc && wvalid) ? 1u : 0u;
     nc_last = nc;
     integrate_lane(L, st, bqacc, jqacc, true);

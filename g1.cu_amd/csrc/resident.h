@@ -2,7 +2,7 @@
 // every control step of one or two worlds, the policy included, with the worlds' state in registers
 // from the first step to the last.
 //
-// For batches of at most two worlds per resident wave of the chip (resident_worlds in g1env.hip). There
+// For batches of at most two worlds per resident wave of the chip (resident_form in g1env.hip). There
 // the work queue of k_rollout has nothing to balance, and its 16-world policy tile costs more than it
 // saves: one wave computes the tile in 43 us while the tile's other seven waves wait for it, each step
 // of all 16 worlds starts when the slowest of the eight pairs has finished the last one, and state,
@@ -13,6 +13,8 @@
 // 3.11 ms, 1024 5.42 -> 3.38, 2048 5.51 -> 3.81, 4096 6.02 -> 4.46; 512-512-256 policy, 4 steps of 512
 // worlds 1.26 -> 0.67, 8 steps of 4096 2.83 -> 1.81. Control steps on given actions (the host step,
 // g1_env_bench_phys) gain the hand-overs between the queue's four items of a step: 3-4% of a launch.
+// Up to 512 worlds a second wave, on a SIMD that would stand idle, takes part of each substep's physics
+// (world_qacc<true>): 16 steps of 256 worlds 1.63 -> 1.50 ms, a step of one world 116 -> 106 us.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -303,10 +305,11 @@ __device__ __forceinline__ int finish_control_step(const PhysArgs& a, const Lane
   return d_flag;
 }
 
-// Enqueue k_resident on the null stream (resident_kernel.hip), with two worlds per wave or one: the
-// policy's rollout of ra.ph.K control steps, or (policy false) K >= 1 control steps on ra.ph.act.
-void launch_resident_kernel(const ResidentArgs& ra, bool policy, bool two);
+// Enqueue k_resident on the null stream (resident_kernel.hip) with one or two worlds per wave, or one
+// world on two waves: the policy's rollout of ra.ph.K control steps, or (policy false) K >= 1 control
+// steps on ra.ph.act.
+void launch_resident_kernel(const ResidentArgs& ra, bool policy, int worlds, int waves);
 // The rollout's function handles (occupancy report).
-const void* resident_kernel_fn(bool two);
+const void* resident_kernel_fn(int worlds, int waves);
 
 }  // namespace g1k

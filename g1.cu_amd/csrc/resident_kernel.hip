@@ -10,14 +10,20 @@ namespace g1k {
 // b and group 0 stores: the second group costs nothing (its lanes would idle), and the wave then runs
 // the contact phases at its own world's contact count instead of the larger of two.
 // kPolicy: the actions come from the policy (K = H steps), else from ph.act.
-template <int kW, bool kPolicy>
-__global__ void __launch_bounds__(kPhysThreads) k_resident(ResidentArgs ra) {
+// kDuo (kW = 1): two waves per world, which share the physics of a substep (world_qacc); both carry the
+// world's state, wave 0 (role 0) runs the policy and stores.
+template <int kW, bool kPolicy, bool kDuo>
+__global__ void __launch_bounds__(kDuo ? 2 * kPhysThreads : kPhysThreads) k_resident(ResidentArgs ra) {
+  static_assert(!kDuo || kW == 1, "two waves per world only with one world per wave");
   __shared__ __align__(16) WorldLds lds[2];
+  __shared__ __align__(16) DuoLds duo[kDuo ? 2 : 1];
+  __shared__ float acts[kGroup];   // kDuo: the policy's actions, from wave 0
+  const int role = kDuo ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
   const int g = group_id(), l = group_lane();
   WorldLds& s = lds[g];
   const int N = ra.ph.N;
   const int w = kW == 2 ? 2 * (int)blockIdx.x + g : (int)blockIdx.x;
-  const bool wvalid = kW == 2 ? w < N : g == 0;
+  const bool wvalid = kW == 2 ? w < N : g == 0 && role == 0;
   const int wc = w < N ? w : N - 1;   // an odd N's last group repeats world N - 1 and stores nothing
   const bool hinge = l >= 2 && l < kNBody;
   LaneState st;
@@ -44,8 +50,16 @@ __global__ void __launch_bounds__(kPhysThreads) k_resident(ResidentArgs ra) {
   for (int k = 0;; ++k) {
     const ResidentArgs& rb = kernarg_reread<ResidentArgs>();
     float act = 0.f;
-    if (kPolicy)   // k == K: the bootstrap value of the state after the last step
-      act = wave_policy<kW>(rb.po, st, pa, rng, rb.ph.seed, rb.ph.N, k, w, wc, wvalid, reinterpret_cast<float*>(lds));
+    if (kPolicy) {   // k == K: the bootstrap value of the state after the last step
+      if (kDuo) __syncthreads();   // wave 1 has read the last substep's results: the policy takes their place
+      if (!kDuo || role == 0)
+        act = wave_policy<kW>(rb.po, st, pa, rng, rb.ph.seed, rb.ph.N, k, w, wc, wvalid, reinterpret_cast<float*>(lds));
+      if (kDuo) {
+        if (role == 0) acts[l] = act;
+        __syncthreads();
+        act = acts[l];
+      }
+    }
     if (k >= K) break;
     // the lane's model constants, formed here (opaque lane index) rather than held across steps
     int lo = l;
@@ -56,7 +70,7 @@ __global__ void __launch_bounds__(kPhysThreads) k_resident(ResidentArgs ra) {
     if (!kPolicy) act = hinge ? a.act[((long)t * a.N + wc) * kAct + l - 2] : 0.f;
     float vx_sum = 0.f, energy = 0.f;
     const SolveParams P{a.pgs, a.mu, true, true};
-    run_substeps(P, s, L, l, wvalid, pd_target(L, act), 0, a.S, st, energy, vx_sum, hcnt);
+    run_substeps<kDuo>(P, s, L, l, wvalid, pd_target(L, act), 0, a.S, st, energy, vx_sum, hcnt, role, duo + (kDuo ? g : 0));
     float r;
     const int done = finish_control_step(a, L, l, wc, t, act, vx_sum, energy, st, pa, step, rng, r);
     if (wvalid && l == 1) {
@@ -79,16 +93,23 @@ __global__ void __launch_bounds__(kPhysThreads) k_resident(ResidentArgs ra) {
   if (a.ncon_hist && l < 9 && hcnt) atomicAdd(&a.ncon_hist[l], (unsigned long long)hcnt);
 }
 
-void launch_resident_kernel(const ResidentArgs& ra, bool policy, bool two) {
-  const dim3 grid((unsigned)(two ? (ra.ph.N + 1) / 2 : ra.ph.N)), block(kPhysThreads);
-  if (policy && two) hipLaunchKernelGGL((k_resident<2, true>), grid, block, 0, 0, ra);
-  else if (policy) hipLaunchKernelGGL((k_resident<1, true>), grid, block, 0, 0, ra);
-  else if (two) hipLaunchKernelGGL((k_resident<2, false>), grid, block, 0, 0, ra);
-  else hipLaunchKernelGGL((k_resident<1, false>), grid, block, 0, 0, ra);
+void launch_resident_kernel(const ResidentArgs& ra, bool policy, int worlds, int waves) {
+  const dim3 grid((unsigned)(worlds == 2 ? (ra.ph.N + 1) / 2 : ra.ph.N)), block(kPhysThreads), pair(2 * kPhysThreads);
+  if (waves == 2) {
+    if (policy) hipLaunchKernelGGL((k_resident<1, true, true>), grid, pair, 0, 0, ra);
+    else hipLaunchKernelGGL((k_resident<1, false, true>), grid, pair, 0, 0, ra);
+  } else if (worlds == 2) {
+    if (policy) hipLaunchKernelGGL((k_resident<2, true, false>), grid, block, 0, 0, ra);
+    else hipLaunchKernelGGL((k_resident<2, false, false>), grid, block, 0, 0, ra);
+  } else {
+    if (policy) hipLaunchKernelGGL((k_resident<1, true, false>), grid, block, 0, 0, ra);
+    else hipLaunchKernelGGL((k_resident<1, false, false>), grid, block, 0, 0, ra);
+  }
 }
 
-const void* resident_kernel_fn(bool two) {
-  return two ? (const void*)k_resident<2, true> : (const void*)k_resident<1, true>;
+const void* resident_kernel_fn(int worlds, int waves) {
+  if (waves == 2) return (const void*)k_resident<1, true, true>;
+  return worlds == 2 ? (const void*)k_resident<2, true, false> : (const void*)k_resident<1, true, false>;
 }
 
 }  // namespace g1k

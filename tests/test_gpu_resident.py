@@ -1,6 +1,6 @@
-"""Launches on batches that fit the chip at one or two worlds per wave (k_resident, up to 4096 worlds) against
-the work-queue form (k_rollout, k_physics), which the fenced hand-over keeps at every size: every output, the
-final state and the contact histogram bit for bit. The two forms share the physics, and the policy's sums run
+"""Launches on batches that fit the chip (k_resident, up to 4096 worlds: one world on two waves up to 512, one
+per wave up to 1024, two per wave) against the work-queue form (k_rollout, k_physics), which the fenced
+hand-over keeps at every size: every output, the final state and the contact histogram bit for bit. The two forms share the physics, and the policy's sums run
 in the same order on the vector ALUs as on v_mfma_f32_16x16x4f32, so the tolerance is zero."""
 import numpy as np
 import pytest
@@ -22,13 +22,13 @@ def _dev(x):
     return torch.from_numpy(np.ascontiguousarray(x)).cuda()
 
 
-# the smallest batches; both sides of one world per wave and of two (odd counts leave half a wave); layers
+# the smallest batches; both sides of two waves per world, of one and of half a wave (odd counts); layers
 # of one to eight row blocks, ragged widths, one to three hidden layers; a horizon of zero
 @pytest.mark.parametrize("N,H,S,hidden,act,given", [
     (1, 3, 10, (256, 256), 0, False), (3, 2, 4, (17, 1), 1, True), (1023, 2, 5, (200, 72), 1, False),
     (1024, 2, 5, (256, 256), 0, True), (1025, 2, 5, (512, 512, 256), 1, True), (2047, 2, 4, (300,), 0, False),
     (4095, 2, 4, (64, 513 - 1, 130), 0, False), (4096, 3, 3, (256, 256), 0, False), (40, 0, 10, (128, 65), 1, False),
-    (130, 12, 10, (256, 256), 0, False)])
+    (130, 12, 10, (256, 256), 0, False), (512, 3, 10, (256, 256), 0, True), (513, 3, 10, (256, 256), 0, True)])
 def test_resident_rollout_equals_work_queue(g1, N, H, S, hidden, act, given):
     import configs
     import torch
@@ -62,7 +62,7 @@ def test_resident_rollout_equals_work_queue(g1, N, H, S, hidden, act, given):
     assert H == 0 or (got[0][5] != 0).any()   # some world finished
 
 
-@pytest.mark.parametrize("N,S", [(1, 10), (33, 1), (1024, 5), (1025, 4), (4095, 3)])
+@pytest.mark.parametrize("N,S", [(1, 10), (33, 1), (512, 10), (513, 10), (1024, 5), (1025, 4), (4095, 3)])
 def test_resident_control_steps_equal_work_queue(g1, N, S):
     """Host steps (observation, reward, done; a finished world restarts) and zero-action physics: the two forms'
     outputs and states bit for bit."""
