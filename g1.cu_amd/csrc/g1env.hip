@@ -763,33 +763,29 @@ static void chunk_schedule(PhysArgs& a, int pgrid, bool one_launch = false) {
   a.nchl = build(big ? 1 : 2, a.cstl);
 }
 
-// The form of a launch: worlds per wave and waves per world of k_resident, or worlds 0: the work queue. One
-// world on two waves while every wave can have a SIMD to itself (512 worlds), one per wave while that
-// holds for them (1024), two per wave while all waves are resident at once (4096). Measured, ms per
-// rollout of the 256-256 policy on two waves, with one world per wave, two, and the queue: 16 steps of 256
-// worlds 1.50, 1.63, 1.83, 2.55; 32 steps of 1024 -,
-// 3.38, 3.85, 5.42; 1536 -, 3.86, 3.87, 5.48; 2048 -, 3.99, 3.81, 5.51; 4096 -, -, 4.46, 6.02; past that
-// a second round of waves would start when the first ends, and the queue spreads the work evenly (8192
-// worlds 7.6). Control steps on given actions, us per 20 steps of standing robots with one, two and the
-// queue: 64 worlds 3452, 3504, 3599; 1024 3615, 3696, 3758; 2048 4162, 3604, 3723; 4096 -, 4176, 4224.
-// An env set to the fenced hand-over keeps the queue, which that mode is about.
-struct ResidentForm { int worlds, waves; };
-static ResidentForm resident_form(const EnvState* E) {
-  if (E->fences) return {0, 0};
-  if (E->N <= E->waves / 4) return {1, 2};
-  if (E->N <= E->waves / 2) return {1, 1};
-  return {E->N <= 2 * E->waves ? 2 : 0, 1};
+// The form of a launch: one world on two waves of k_resident while all of them are resident at once (1024
+// worlds), two worlds per wave while that holds for those (4096), and the work queue past that, where a
+// second round of waves would start when the first ends and the queue spreads the work evenly. Measured,
+// ms per rollout of the 256-256 policy with one world on two waves, one per wave, two per wave, and the
+// queue: 16 steps of 256 worlds 1.50, 1.63, 1.83, 2.55; 768 1.64, 1.75, 1.96, -; 32 steps of 1024 3.22,
+// 3.34, 3.85, 5.42; 1536 -, 3.86, 3.87, 5.48; 2048 -, 3.99, 3.81, 5.51; 4096 -, -, 4.46, 6.02 (8192 on the
+// queue 7.6). Five control steps on given actions, us, of 1024 standing worlds: 796, 837, 850, 930. An
+// env set to the fenced hand-over keeps the queue, which that mode is about.
+enum class Form { kQueue, kDuo, kPair };
+static Form launch_form(const EnvState* E) {
+  if (E->fences || E->N > 2 * E->waves) return Form::kQueue;
+  return E->N <= E->waves / 2 ? Form::kDuo : Form::kPair;
 }
 
 // Enqueue one physics launch on the null stream; the queue state (flag base, counter row) advances
 // on the host in launch order, which is the stream's execution order.
 static void launch_physics(EnvState* E, PhysArgs& a) {
   if (a.K <= 0) fail("physics launch: K must be positive");
-  const ResidentForm form = resident_form(E);
-  if (form.worlds) {
+  const Form form = launch_form(E);
+  if (form != Form::kQueue) {
     ResidentArgs ra{};
     ra.ph = a;
-    launch_resident_kernel(ra, false, form.worlds, form.waves);
+    launch_resident_kernel(ra, false, form == Form::kDuo);
     HIPCHECK(hipGetLastError());
     return;
   }
@@ -821,7 +817,7 @@ static void check_queue(EnvState* E) { check_queue_error(*(volatile int*)E->qerr
 // The one-launch rollout runs policies of two hidden layers of at most 256 units each on the
 // register-resident tile (policy_tile, at 256-256 with zero padding) and every other accepted shape
 // (1..3 hidden layers of at most 512 units) on the wide tile (policy_tile_wide, activations staged
-// in global memory); small batches of either kind run resident waves (resident_form). The split form
+// in global memory); small batches of either kind run resident waves (launch_form). The split form
 // (policy and physics launches per control step) remains for g1_env_set_fused(h, 0) and for
 // g1_rollout_noalloc with a wide shape (the wide tile's activation buffers are allocated by the library).
 static bool narrow_shape(const PolicyShape& sh) {
@@ -861,7 +857,7 @@ static void pack_wide(EnvState* E, const float* W, const float* mean, const floa
 }
 
 // The whole rollout as one k_resident launch on the null stream; wp as in rollout_fused.
-static void rollout_resident(EnvState* E, ResidentForm form, int H, const float* W, const float* mean, const float* var,
+static void rollout_resident(EnvState* E, Form form, int H, const float* W, const float* mean, const float* var,
                              float* O, float* A, float* LP, float* V, float* R, float* D, float* Vlast,
                              const float* act_noise, const float* reset_noise, float* wp, long wp_cap) {
   const WideLayout wl = wide_layout(E->shape.nl, E->shape.hid, E->shape.act);
@@ -874,7 +870,7 @@ static void rollout_resident(EnvState* E, ResidentForm form, int H, const float*
   ra.po = TileArgs{Wt, TileLayout{}, act_noise, O, A, LP, V, Vlast, H, 1, wl, nullptr};
   const bool prof = E->prof_on != 0 && !wp;
   if (prof) prof_mark(E->ev_phys, E->n_phys);
-  launch_resident_kernel(ra, true, form.worlds, form.waves);
+  launch_resident_kernel(ra, true, form == Form::kDuo);
   HIPCHECK(hipGetLastError());
   if (prof) prof_mark(E->ev_phys, E->n_phys);
 }
@@ -935,8 +931,8 @@ static void rollout_impl(EnvState* E, int H, const float* W, const float* mean, 
   check_queue(E);
   if (H < 0) H = 0;   // no control step; the bootstrap value is still computed (as the reference's k_rollout)
   if (E->fused && fused_shape(E->shape, wp != nullptr)) {
-    const ResidentForm form = resident_form(E);
-    if (form.worlds) {
+    const Form form = launch_form(E);
+    if (form != Form::kQueue) {
       rollout_resident(E, form, H, W, mean, var, O, A, LP, V, R, D, Vlast, act_noise, reset_noise, wp, wp_cap);
       return;
     }
@@ -1221,9 +1217,8 @@ void g1_occupancy_report(void) {
   struct { const char* nm; const void* fn; int threads; size_t smem; } ks[] = {
       {"k_rollout", rollout_kernel_fn(false), kPhysThreads, 0},
       {"k_rollout (wide)", rollout_kernel_fn(true), kPhysThreads, 0},
-      {"k_resident (1/2)", resident_kernel_fn(1, 2), 2 * kPhysThreads, 0},
-      {"k_resident (1)", resident_kernel_fn(1, 1), kPhysThreads, 0},
-      {"k_resident (2)", resident_kernel_fn(2, 1), kPhysThreads, 0},
+      {"k_resident (duo)", resident_kernel_fn(true), 2 * kPhysThreads, 0},
+      {"k_resident", resident_kernel_fn(false), kPhysThreads, 0},
       {"k_physics", (const void*)k_physics, kPhysThreads, 0},
       {"k_policy", (const void*)k_policy, kPolicyThreads, policy_smem(PolicyShape{2, {256, 256, 0, 0}, 0})},
       {"k_probe", (const void*)k_probe, kPhysThreads, 0}};

@@ -620,7 +620,8 @@ __device__ __forceinline__ void base_solve(const WorldLds& s, const float (&xb)[
 }
 
 // Ordering point between the phases of world_qacc, whose callers run it in workgroups of one wave
-// (k_physics, k_rollout, k_resident, k_probe: 64 threads). A wave's LDS accesses are performed in
+// (k_physics, k_rollout, k_resident, k_probe: 64 threads;
+// k_resident with two waves per world adds block barriers between them, duo_sync). A wave's LDS accesses are performed in
 // program order, so a wavefront-scope fence (the compiler keeps the accesses in order; no instruction)
 // is all a hand-over through LDS between its lanes needs; __syncthreads() adds an lgkmcnt(0) drain of
 // every outstanding LDS access at each phase boundary: the training rollout 10.50 -> 10.43 ms when the

@@ -1,20 +1,20 @@
-// resident.h -- a wave that keeps its worlds for a whole launch (k_resident, resident_kernel.hip):
-// every control step of one or two worlds, the policy included, with the worlds' state in registers
-// from the first step to the last.
+// resident.h -- waves that keep their worlds for a whole launch (k_resident, resident_kernel.hip): every
+// control step of two worlds on one wave, or of one world on two waves, the policy included, with the
+// worlds' state in registers from the first step to the last.
 //
-// For batches of at most two worlds per resident wave of the chip (resident_form in g1env.hip). There
+// For batches of at most two worlds per resident wave of the chip (launch_form in g1env.hip). There
 // the work queue of k_rollout has nothing to balance, and its 16-world policy tile costs more than it
 // saves: one wave computes the tile in 43 us while the tile's other seven waves wait for it, each step
 // of all 16 worlds starts when the slowest of the eight pairs has finished the last one, and state,
-// actions and flags cross the L2 between the waves. Here nothing is waited for but the wave's own work.
-// Bound by one wave's instruction issue (about one per four cycles): a substep takes 8.6 us with one
-// world per wave and 9.5 us with two (a wave alone on its SIMD), the rest of a control step 15 us, of
-// which the 256-256 policy is about 10. Rollouts of 32 control steps against the queue: 32 worlds 4.36 ->
-// 3.11 ms, 1024 5.42 -> 3.38, 2048 5.51 -> 3.81, 4096 6.02 -> 4.46; 512-512-256 policy, 4 steps of 512
-// worlds 1.26 -> 0.67, 8 steps of 4096 2.83 -> 1.81. Control steps on given actions (the host step,
-// g1_env_bench_phys) gain the hand-overs between the queue's four items of a step: 3-4% of a launch.
-// Up to 512 worlds a second wave, on a SIMD that would stand idle, takes part of each substep's physics
-// (world_qacc<true>): 16 steps of 256 worlds 1.63 -> 1.50 ms, a step of one world 116 -> 106 us.
+// actions and flags cross the L2 between the waves. Here nothing is waited for but the world's own work.
+// Bound by one wave's instruction issue (about one per four cycles): 8 to 9 us per substep, and 13 us for
+// the rest of a control step, of which the 256-256 policy is 12 (its weights' way from the L2). Up to
+// 1024 worlds a second wave takes part of each substep's physics (world_qacc<true>) on a SIMD that would
+// stand idle or carry one wave. Rollouts against the queue: 32 steps of 32 worlds 4.36 -> 2.9 ms, 1024 5.42
+// -> 3.22, 2048 5.51 -> 3.75, 4096 6.02 -> 4.4; 512-512-256 policy, 4 steps of 512 worlds 1.26 -> 0.63, 8
+// steps of 4096 2.83 -> 1.81. Control steps on given actions (the host step, g1_env_bench_phys): one
+// world, a step 149 -> 106 us (of it 27 the outputs' way to the host), 5 steps of 1024 standing worlds 930
+// -> 796.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -305,11 +305,11 @@ __device__ __forceinline__ int finish_control_step(const PhysArgs& a, const Lane
   return d_flag;
 }
 
-// Enqueue k_resident on the null stream (resident_kernel.hip) with one or two worlds per wave, or one
-// world on two waves: the policy's rollout of ra.ph.K control steps, or (policy false) K >= 1 control
-// steps on ra.ph.act.
-void launch_resident_kernel(const ResidentArgs& ra, bool policy, int worlds, int waves);
+// Enqueue k_resident on the null stream (resident_kernel.hip) with one world on two waves (duo) or two
+// worlds per wave: the policy's rollout of ra.ph.K control steps, or (policy false) K >= 1 control steps
+// on ra.ph.act.
+void launch_resident_kernel(const ResidentArgs& ra, bool policy, bool duo);
 // The rollout's function handles (occupancy report).
-const void* resident_kernel_fn(int worlds, int waves);
+const void* resident_kernel_fn(bool duo);
 
 }  // namespace g1k

@@ -1,20 +1,19 @@
-// resident_kernel.hip -- k_resident: a whole rollout, or K control steps on given actions, with one or two
-// worlds per wave (resident.h).
+// resident_kernel.hip -- k_resident: a whole rollout, or K control steps on given actions, with two worlds
+// per wave or one world on two waves (resident.h).
 #include <hip/hip_runtime.h>
 
 #include "resident.h"
 
 namespace g1k {
 
-// kW: worlds per wave. With two, group g of block b has world 2 b + g; with one, both groups carry world
-// b and group 0 stores: the second group costs nothing (its lanes would idle), and the wave then runs
-// the contact phases at its own world's contact count instead of the larger of two.
-// kPolicy: the actions come from the policy (K = H steps), else from ph.act.
-// kDuo (kW = 1): two waves per world, which share the physics of a substep (world_qacc); both carry the
-// world's state, wave 0 (role 0) runs the policy and stores.
-template <int kW, bool kPolicy, bool kDuo>
+// kDuo: one world on two waves, which share the physics of a substep (world_qacc); both carry the world's
+// state, wave 0 (role 0) runs the policy and stores. Else two worlds on one wave: group g of block b has
+// world 2 b + g. With one world both groups of a wave carry it and group 0 stores: the second group costs
+// nothing (its lanes would idle), and the contact phases run at the world's own contact count instead of
+// the larger of two. kPolicy: the actions come from the policy (K = H steps), else from ph.act.
+template <bool kDuo, bool kPolicy>
 __global__ void __launch_bounds__(kDuo ? 2 * kPhysThreads : kPhysThreads) k_resident(ResidentArgs ra) {
-  static_assert(!kDuo || kW == 1, "two waves per world only with one world per wave");
+  constexpr int kW = kDuo ? 1 : 2;   // worlds per wave
   __shared__ __align__(16) WorldLds lds[2];
   __shared__ __align__(16) DuoLds duo[kDuo ? 2 : 1];
   __shared__ float acts[kGroup];   // kDuo: the policy's actions, from wave 0
@@ -93,23 +92,16 @@ __global__ void __launch_bounds__(kDuo ? 2 * kPhysThreads : kPhysThreads) k_resi
   if (a.ncon_hist && l < 9 && hcnt) atomicAdd(&a.ncon_hist[l], (unsigned long long)hcnt);
 }
 
-void launch_resident_kernel(const ResidentArgs& ra, bool policy, int worlds, int waves) {
-  const dim3 grid((unsigned)(worlds == 2 ? (ra.ph.N + 1) / 2 : ra.ph.N)), block(kPhysThreads), pair(2 * kPhysThreads);
-  if (waves == 2) {
-    if (policy) hipLaunchKernelGGL((k_resident<1, true, true>), grid, pair, 0, 0, ra);
-    else hipLaunchKernelGGL((k_resident<1, false, true>), grid, pair, 0, 0, ra);
-  } else if (worlds == 2) {
-    if (policy) hipLaunchKernelGGL((k_resident<2, true, false>), grid, block, 0, 0, ra);
-    else hipLaunchKernelGGL((k_resident<2, false, false>), grid, block, 0, 0, ra);
-  } else {
-    if (policy) hipLaunchKernelGGL((k_resident<1, true, false>), grid, block, 0, 0, ra);
-    else hipLaunchKernelGGL((k_resident<1, false, false>), grid, block, 0, 0, ra);
-  }
+void launch_resident_kernel(const ResidentArgs& ra, bool policy, bool duo) {
+  const dim3 grid((unsigned)(duo ? ra.ph.N : (ra.ph.N + 1) / 2)), block(duo ? 2 * kPhysThreads : kPhysThreads);
+  if (duo && policy) hipLaunchKernelGGL((k_resident<true, true>), grid, block, 0, 0, ra);
+  else if (duo) hipLaunchKernelGGL((k_resident<true, false>), grid, block, 0, 0, ra);
+  else if (policy) hipLaunchKernelGGL((k_resident<false, true>), grid, block, 0, 0, ra);
+  else hipLaunchKernelGGL((k_resident<false, false>), grid, block, 0, 0, ra);
 }
 
-const void* resident_kernel_fn(int worlds, int waves) {
-  if (waves == 2) return (const void*)k_resident<1, true, true>;
-  return worlds == 2 ? (const void*)k_resident<2, true, false> : (const void*)k_resident<1, true, false>;
+const void* resident_kernel_fn(bool duo) {
+  return duo ? (const void*)k_resident<true, true> : (const void*)k_resident<false, true>;
 }
 
 }  // namespace g1k

@@ -1,5 +1,5 @@
-"""Launches on batches that fit the chip (k_resident, up to 4096 worlds: one world on two waves up to 512, one
-per wave up to 1024, two per wave) against the work-queue form (k_rollout, k_physics), which the fenced
+"""Launches on batches that fit the chip (k_resident, up to 4096 worlds: one world on two waves up to 1024,
+then two per wave) against the work-queue form (k_rollout, k_physics), which the fenced
 hand-over keeps at every size: every output, the final state and the contact histogram bit for bit. The two forms share the physics, and the policy's sums run
 in the same order on the vector ALUs as on v_mfma_f32_16x16x4f32, so the tolerance is zero."""
 import numpy as np
@@ -22,7 +22,7 @@ def _dev(x):
     return torch.from_numpy(np.ascontiguousarray(x)).cuda()
 
 
-# the smallest batches; both sides of two waves per world, of one and of half a wave (odd counts); layers
+# the smallest batches; both sides of two waves per world and of two worlds per wave (odd counts); layers
 # of one to eight row blocks, ragged widths, one to three hidden layers; a horizon of zero
 @pytest.mark.parametrize("N,H,S,hidden,act,given", [
     (1, 3, 10, (256, 256), 0, False), (3, 2, 4, (17, 1), 1, True), (1023, 2, 5, (200, 72), 1, False),
