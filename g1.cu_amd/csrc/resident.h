@@ -7,12 +7,13 @@
 // saves: one wave computes the tile in 43 us while the tile's other seven waves wait for it, each step
 // of all 16 worlds starts when the slowest of the eight pairs has finished the last one, and state,
 // actions and flags cross the L2 between the waves. Here nothing is waited for but the world's own work.
-// Bound by one wave's instruction issue (about one per four cycles): 8 to 9 us per substep, and 13 us for
-// the rest of a control step, of which the 256-256 policy is 12 (its weights' way from the L2). Up to
-// 1024 worlds a second wave takes part of each substep's physics (world_qacc<true>) on a SIMD that would
-// stand idle or carry one wave. Rollouts against the queue: 32 steps of 32 worlds 4.36 -> 2.9 ms, 1024 5.42
-// -> 3.22, 2048 5.51 -> 3.75, 4096 6.02 -> 4.4; 512-512-256 policy, 4 steps of 512 worlds 1.26 -> 0.63, 8
-// steps of 4096 2.83 -> 1.81. Control steps on given actions (the host step, g1_env_bench_phys): one
+// Bound by one wave's instruction issue (about one per four cycles): 8 to 9 us per substep, and 10 to 13 us
+// for the rest of a control step, most of it the 256-256 policy (its weights' way from the L2). Up to 1024
+// worlds a second wave, on a SIMD that would stand idle or carry one wave, takes part of each substep's
+// physics (world_qacc<true>) and half of the policy's rows (16 steps of 256 worlds 1.51 -> 1.47 ms by the
+// latter; 4 steps of 512 with the 512-512-256 policy 0.63 -> 0.57). Rollouts against the queue: 16 steps of
+// 256 worlds 2.55 -> 1.47 ms, 32 steps of 1024 5.42 -> 3.18, 2048 5.51 -> 3.75, 4096 6.02 -> 4.4; 512-512-256
+// policy, 4 steps of 512 worlds 1.26 -> 0.57, 8 steps of 4096 2.83 -> 1.81. Control steps on given actions (the host step, g1_env_bench_phys): one
 // world, a step 149 -> 106 us (of it 27 the outputs' way to the host), 5 steps of 1024 standing worlds 930
 // -> 796.
 #pragma once
@@ -154,16 +155,21 @@ __device__ __forceinline__ void net_rows(const float4* W, const float* bias, int
 // Policy of control step t for the wave's worlds (t == a.H: the bootstrap value only): observation,
 // normalisation, MLP, sampling and log-probability, with the values of the policy tiles (rollout.h) bit
 // for bit. The worlds' state is in the lanes (st, pa, rng); w: the group's world, wvalid: its lanes store.
-// Returns the lane's own action (hinge lanes; t < a.H). lds: kNetLds floats.
-template <int kW>
+// Returns the lane's own action (hinge lanes; t < a.H). lds: kNetLds floats. kDuo: both waves of the world
+// call it; wave 0 forms the observation, the head and the outputs, and each takes half of a hidden layer's
+// rows, with a block barrier after the observation and after each layer (nl + 1 on either wave): one
+// wave's loads reach about 22 bytes per clock of the L2's way to its CU, two twice that. (Returns 0 on
+// wave 1.)
+template <int kW, bool kDuo>
 __device__ __forceinline__ float wave_policy(const TileArgs& a, const LaneState& st, float pa, unsigned rng,
                                              unsigned long long seed, int N, int t, int w, int wc, bool wvalid,
-                                             float* lds) {
+                                             float* lds, int role) {
   int lane = threadIdx.x & 63;
   __asm__ volatile("" : "+v"(lane));
   const int l = lane & 31, v = kW == 2 ? lane >> 5 : 0;
   const WideLayout& T = a.wl;
   float* const mine = lds + v * kNetWorld;
+  if (!kDuo || role == 0) {
   // ---- observation (raw to O) and frozen normalisation: the lanes put their world's features into the
   // second buffer, and lane l takes features l, 32 + l, 64 + l, 96 + l from there
   const float* const nrm = a.Wt + T.nrm_off;
@@ -201,7 +207,9 @@ __device__ __forceinline__ float wave_policy(const TileArgs& a, const LaneState&
     }
   }
   wave_sync();
-  // ---- hidden layers: four row blocks (256 rows) at a time, then what is left
+  }
+  if (kDuo) __syncthreads();
+  // ---- hidden layers: four row blocks (256 rows) at a time, then two, then one
   const float4* const W = reinterpret_cast<const float4*>(a.Wt);
 #pragma unroll 1
   for (int ly = 0; ly < T.nl; ++ly) {
@@ -210,13 +218,20 @@ __device__ __forceinline__ float wave_policy(const TileArgs& a, const LaneState&
     const float4* const Wl = W + T.woff[ly] / 4;
     const float* const bl = a.Wt + T.boff[ly];
     const int nT = T.nT[ly], nQ = T.nQ[ly];
-    int T0 = 0;
+    const int half = kDuo ? (nT / 4 + 1) / 2 * 4 : nT;   // a wave's tiles (whole row blocks)
+    int T0 = kDuo && role != 0 ? half : 0;
+    const int T1 = kDuo && role == 0 ? half : nT;
 #pragma unroll 1
-    for (; T0 + 16 <= nT; T0 += 16) net_rows<kW, 4>(Wl, bl, nQ, T0, x, out, T.act, lane);
-#pragma unroll 1
-    for (; T0 < nT; T0 += 4) net_rows<kW, 1>(Wl, bl, nQ, T0, x, out, T.act, lane);
-    wave_sync();
+    for (; T0 + 16 <= T1; T0 += 16) net_rows<kW, 4>(Wl, bl, nQ, T0, x, out, T.act, lane);
+    if (T0 + 8 <= T1) {
+      net_rows<kW, 2>(Wl, bl, nQ, T0, x, out, T.act, lane);
+      T0 += 8;
+    }
+    if (T0 < T1) net_rows<kW, 1>(Wl, bl, nQ, T0, x, out, T.act, lane);
+    if (kDuo) __syncthreads();
+    else wave_sync();
   }
+  if (kDuo && role != 0) return 0.f;
   // ---- head: lane (v, 16 ht + j) has row i = 16 ht + j of world v (mu 0..28, value 29)
   float hd[1][1];
   net_pass<1, 1, 4, true>(W + T.woff[T.nl] / 4, a.Wt + T.boff[T.nl], T.nQ[T.nl], 0, mine + (T.nl & 1) * kNetBuf, lane, hd);

@@ -7,7 +7,7 @@
 namespace g1k {
 
 // kDuo: one world on two waves, which share the physics of a substep (world_qacc); both carry the world's
-// state, wave 0 (role 0) runs the policy and stores. Else two worlds on one wave: group g of block b has
+// state, wave 0 (role 0) stores. Else two worlds on one wave: group g of block b has
 // world 2 b + g. With one world both groups of a wave carry it and group 0 stores: the second group costs
 // nothing (its lanes would idle), and the contact phases run at the world's own contact count instead of
 // the larger of two. kPolicy: the actions come from the policy (K = H steps), else from ph.act.
@@ -51,8 +51,8 @@ __global__ void __launch_bounds__(kDuo ? 2 * kPhysThreads : kPhysThreads) k_resi
     float act = 0.f;
     if (kPolicy) {   // k == K: the bootstrap value of the state after the last step
       if (kDuo) __syncthreads();   // wave 1 has read the last substep's results: the policy takes their place
-      if (!kDuo || role == 0)
-        act = wave_policy<kW>(rb.po, st, pa, rng, rb.ph.seed, rb.ph.N, k, w, wc, wvalid, reinterpret_cast<float*>(lds));
+      act = wave_policy<kW, kDuo>(rb.po, st, pa, rng, rb.ph.seed, rb.ph.N, k, w, wc, wvalid,
+                                  reinterpret_cast<float*>(lds), role);
       if (kDuo) {
         if (role == 0) acts[l] = act;
         __syncthreads();
