@@ -619,14 +619,14 @@ __device__ __forceinline__ void base_solve(const WorldLds& s, const float (&xb)[
   for (int i = 0; i < 6; ++i) a1[i] = sbase_col(i, S3, qdd);
 }
 
-// Ordering point between the phases of world_qacc, whose callers run it in workgroups of one wave
-// (k_physics, k_rollout, k_resident, k_probe: 64 threads;
-// k_resident with two waves per world adds block barriers between them, duo_sync). A wave's LDS accesses are performed in
-// program order, so a wavefront-scope fence (the compiler keeps the accesses in order; no instruction)
-// is all a hand-over through LDS between its lanes needs; __syncthreads() adds an lgkmcnt(0) drain of
-// every outstanding LDS access at each phase boundary: the training rollout 10.50 -> 10.43 ms when the
-// fence came in; k_physics and k_probe followed later (50 steps of 8192 standing worlds 19.00 -> 18.93
-// ms, a host step of 8192 485 -> 480 us, ten contact-free substeps 181.0 -> 179.9 us).
+// Ordering point between the phases of world_qacc within a wave (the workgroups of k_physics, k_rollout,
+// k_probe and k_resident are one wave; where k_resident has two per world, duo_sync hands over between
+// them). A wave's LDS accesses are performed in program order, so a wavefront-scope fence (the compiler
+// keeps the accesses in order; no instruction) is all a hand-over through LDS between its lanes needs;
+// __syncthreads() adds an lgkmcnt(0) drain of every outstanding LDS access at each phase boundary: the
+// training rollout 10.50 -> 10.43 ms when the fence came in; k_physics and k_probe followed later (50 steps
+// of 8192 standing worlds 19.00 -> 18.93 ms, a host step of 8192 485 -> 480 us, ten contact-free substeps
+// 181.0 -> 179.9 us).
 __device__ __forceinline__ void wave_sync() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
 // The chain layout's stores without a lane test (the factor, the force gather, the RNE staging): a
