@@ -473,7 +473,7 @@ struct SolveParams {
 // count nefc_max is a multiple of 4), so the sweep tests nefc_max at every fourth row and branches
 // once to its end. W: the rows a world can hold in this wave (nefc_max <= W): lane i holds row i
 // and the change is broadcast over its first 16-lane row (16) or its quad (4); for W = 32 see
-// pgs_row_pair.
+// pgs_rows_pair.
 //
 // A row in VALU code (W = 16): fn = max(-r, 0), d = fn - f, f = fn on row II's lanes (a lane
 // mask), then r += a d with d taken from lane II of the 16-lane row by DPP row_newbcast inside the
@@ -488,6 +488,9 @@ struct SolveParams {
 // 8192 standing worlds 20.79 -> 20.58 ms). max(-r, 0) is 0 for a NaN r (the quiet NaNs of arithmetic), as t > 0 ? t : 0 is.
 // `lanes`: the row's lanes, lane II of every 16-lane row (from an opaque base in each sweep: as 32
 // constants the compiler holds the masks in scalar registers across the sweep loop and spills them).
+// A block writes f, the residuals and the mask in its first row and reads the later rows' entries after
+// that, so those operands are early-clobbered: else an entry that holds the value of one of them at the
+// block's start may be given its register.
 
 // Lane 0 of every 16-lane row: the lanes of a sweep's first row.
 __device__ __forceinline__ unsigned long long pgs_lanes0() {
@@ -523,7 +526,7 @@ __device__ __forceinline__ void pgs_rows(const float (&A)[kMaxEfc], int l, unsig
   } else {
     float fn, d;
     __asm__(G1_PGS_ROW("%5", "%9") G1_PGS_ROW("%6", "%10") G1_PGS_ROW("%7", "%11") G1_PGS_ROW("%8", "%12")
-            : "+v"(fi), "+v"(ri), "=&v"(fn), "=&v"(d), "+s"(lanes)
+            : "+&v"(fi), "+&v"(ri), "=&v"(fn), "=&v"(d), "+&s"(lanes)
             : "v"(A[II]), "v"(A[II + 1]), "v"(A[II + 2]), "v"(A[II + 3]), "n"(II), "n"(II + 1), "n"(II + 2), "n"(II + 3)
             : "scc");
   }
@@ -562,7 +565,7 @@ __device__ __forceinline__ void pgs_rows_pair(const float (&A)[kMaxEfc], const f
   float fn, d;
   __asm__(G1_PGS_ROW("%6", "%10", "%14") G1_PGS_ROW("%7", "%11", "%15") G1_PGS_ROW("%8", "%12", "%16")
           G1_PGS_ROW("%9", "%13", "%17")
-          : "+v"(f), "+v"(r), "+v"(ro), "=&v"(fn), "=&v"(d), "+s"(lanes)
+          : "+&v"(f), "+&v"(r), "+&v"(ro), "=&v"(fn), "=&v"(d), "+&s"(lanes)
           : "v"(A[II]), "v"(A[II + 1]), "v"(A[II + 2]), "v"(A[II + 3]), "v"(B[II]), "v"(B[II + 1]), "v"(B[II + 2]),
             "v"(B[II + 3]), "n"(II & 15), "n"((II & 15) + 1), "n"((II & 15) + 2), "n"((II & 15) + 3)
           : "scc");
