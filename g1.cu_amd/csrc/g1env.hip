@@ -79,8 +79,7 @@ __global__ void __launch_bounds__(kPhysThreads) k_physics(PhysArgs a) {
   };
   set_queue(q);
   unsigned hcnt = 0;   // lane q < 9 counts substeps with q contacts
-  if (a.xlocal && threadIdx.x == 0 && xcc_id() != q % kXcds)
-    __hip_atomic_store(a.qerr, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (a.xlocal && threadIdx.x == 0 && xcc_id() != q % kXcds) report_queue_error(a.qerr, 2);
 
 #pragma unroll 1
   for (;;) {

@@ -65,6 +65,13 @@ __device__ __forceinline__ T ld_l2(const T* p) {
 // xlocal the hand-over uses agent-scope release/acquire fences, which also write back and
 // invalidate the L2 (correct on any placement, much slower).
 
+// A queue error into the env's error word. The word lies in pinned host memory, which the host also reads
+// while the kernel runs, so the store is at system scope (an agent-scope one is ordered for this GPU only).
+// Called by one lane.
+__device__ __forceinline__ void report_queue_error(int* qerr, int code) {
+  __hip_atomic_store(qerr, code, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Wait until *flag >= want (wrap-safe). A wait that exceeds kSpinLimit polls sets qerr = 1 and
 // returns: every item waited for was claimed earlier by a running wave, so a wait ends unless the
 // hardware stalls; the error makes the next synchronising call exit.
@@ -75,7 +82,7 @@ __device__ __forceinline__ void wait_flag(const unsigned* flag, unsigned want, i
     const unsigned f = __builtin_amdgcn_readfirstlane(ld_l2(flag));
     if ((int)(f - want) >= 0) break;
     if (++spins > kSpinLimit) {
-      if (threadIdx.x == 0) __hip_atomic_store(qerr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (threadIdx.x == 0) report_queue_error(qerr, 1);
       break;
     }
     __builtin_amdgcn_s_sleep(2);

@@ -36,8 +36,7 @@ __global__ void __launch_bounds__(kPhysThreads) k_rollout(RolloutArgs ra) {
   };
   set_queue(q);
   unsigned hcnt = 0;
-  if (a.xlocal && threadIdx.x == 0 && xcc_id() != q % kXcds)
-    __hip_atomic_store(a.qerr, 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (a.xlocal && threadIdx.x == 0 && xcc_id() != q % kXcds) report_queue_error(a.qerr, 2);
   float* scratch_lds = reinterpret_cast<float*>(lds_raw);
   // policy of step t on tile u of queue qq (its np pairs complete through step t - 1)
   auto policy = [&](int qq, int u, int np, int t) {
