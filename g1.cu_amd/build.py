@@ -96,8 +96,9 @@ def build(verbose=False):
     with open(RESOURCES, "w") as f:
         json.dump(resources, f, indent=1, sort_keys=True)
     for fn, r in resources.items():
-        if ("k_rollout" in fn or "k_physics" in fn) and (r.get("Occupancy", 0) < 2 or r.get("ScratchSize", 0)):
-            sys.stderr.write(f"WARNING: {fn}: {r} (the persistent kernels are sized for 2 waves/SIMD, no scratch)\n")
+        sized = any(k in fn for k in ("k_rollout", "k_physics", "k_resident"))
+        if sized and (r.get("Occupancy", 0) < 2 or r.get("ScratchSize", 0)):
+            sys.stderr.write(f"WARNING: {fn}: {r} (the kernels that keep the chip are sized for 2 waves/SIMD, no scratch)\n")
     return OUT
 
 

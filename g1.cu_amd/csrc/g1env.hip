@@ -572,8 +572,9 @@ struct EnvState {
   float *qacc_e, *qacc_vx;
   unsigned qdone;   // value of every pair flag after the launches enqueued so far
   int qpar;         // counter row of the next launch
-  int waves;        // blocks of k_physics resident on the chip, a multiple of kQueues
-  int pgrid;        // persistent grid: those blocks, no more than the pairs need
+  int pgrid;        // persistent grid: the blocks of k_physics resident on the chip, a multiple of kQueues,
+                    //   no more than the pairs need
+  int duo_worlds, pair_worlds;   // worlds that k_resident holds on the chip at once: on two waves each, two per wave
   int xlocal;       // blocks land on XCD blockIdx % kXcds (measured at creation)
   int fences;       // 1: hand over state with agent-scope fences even where xlocal holds
   // one-launch rollout (k_rollout): policy tiles' flags, their completed-step count, packed weights
@@ -770,10 +771,11 @@ static void chunk_schedule(PhysArgs& a, int pgrid, bool one_launch = false) {
 // 3.34, 3.85, 5.42; 1536 -, 3.86, 3.87, 5.48; 2048 -, 3.99, 3.81, 5.51; 4096 -, -, 4.46, 6.02 (8192 on the
 // queue 7.6). Five control steps on given actions, us, of 1024 standing worlds: 796, 837, 850, 930. An
 // env set to the fenced hand-over keeps the queue, which that mode is about.
-enum class Form { kQueue, kDuo, kPair };
+enum class Form { kQueue, kDuo, kPair };   // (values: g1_env_launch_form)
 static Form launch_form(const EnvState* E) {
-  if (E->fences || E->N > 2 * E->waves) return Form::kQueue;
-  return E->N <= E->waves / 2 ? Form::kDuo : Form::kPair;
+  if (E->fences) return Form::kQueue;
+  if (E->N <= E->duo_worlds) return Form::kDuo;
+  return E->N <= E->pair_worlds ? Form::kPair : Form::kQueue;
 }
 
 // Enqueue one physics launch on the null stream; the queue state (flag base, counter row) advances
@@ -1023,8 +1025,17 @@ void* g1_env_create(int N, int substeps, int pgs_iters, unsigned long seed) {
     int cap = (cus * (per_cu > 0 ? per_cu : 1)) / kQueues * kQueues;
     if (cap < kQueues) cap = kQueues;
     const int need = (npairs + kQueues - 1) / kQueues * kQueues;
-    E->waves = cap;
     E->pgrid = need < cap ? need : cap;
+    // one world per block on two waves, two on one wave; both instantiations of a form have to be resident
+    auto resident_blocks = [&](bool duo) {
+      int n[2];
+      for (int policy = 0; policy < 2; ++policy)
+        HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n[policy], resident_kernel_fn(policy, duo),
+                                                              resident_threads(duo), 0));
+      return cus * std::min(n[0], n[1]);
+    };
+    E->duo_worlds = resident_blocks(true);
+    E->pair_worlds = 2 * resident_blocks(false);
     // placement of the blocks on the XCDs: round-robin lets each queue hand over state in one L2
     int* dx = nullptr;
     HIPCHECK(hipMalloc(&dx, (size_t)E->pgrid * sizeof(int)));
@@ -1080,7 +1091,7 @@ void g1_env_destroy(void* h) {
 // fit the chip at once, whose step is a matter of tens of microseconds of copies and synchronisations
 // (us per step, through device memory and directly: 1 world 149, 122; 1024 282, 181; 4096 330, 269). Of
 // larger outputs the host copies one part while the next is transferred (8192 worlds 479; directly 513).
-static bool direct_outputs(const EnvState* E) { return E->N <= 2 * E->waves; }
+static bool direct_outputs(const EnvState* E) { return E->N <= E->pair_worlds; }
 
 // The observations, and with rew the rewards and done flags, from the device's [obs | reward | done] to
 // the caller's arrays, through the pinned staging in chunks of worlds: the host copy of one chunk overlaps
@@ -1216,8 +1227,8 @@ void g1_occupancy_report(void) {
   struct { const char* nm; const void* fn; int threads; size_t smem; } ks[] = {
       {"k_rollout", rollout_kernel_fn(false), kPhysThreads, 0},
       {"k_rollout (wide)", rollout_kernel_fn(true), kPhysThreads, 0},
-      {"k_resident (duo)", resident_kernel_fn(true), 2 * kPhysThreads, 0},
-      {"k_resident", resident_kernel_fn(false), kPhysThreads, 0},
+      {"k_resident (duo)", resident_kernel_fn(true, true), resident_threads(true), 0},
+      {"k_resident", resident_kernel_fn(true, false), resident_threads(false), 0},
       {"k_physics", (const void*)k_physics, kPhysThreads, 0},
       {"k_policy", (const void*)k_policy, kPolicyThreads, policy_smem(PolicyShape{2, {256, 256, 0, 0}, 0})},
       {"k_probe", (const void*)k_probe, kPhysThreads, 0}};
@@ -1325,6 +1336,8 @@ int g1_env_set_fused(void* h, int on) {
   E->fused = on;
   return (on && !fused_shape(E->shape, false)) ? 1 : 0;
 }
+
+int g1_env_launch_form(void* h) { return (int)launch_form((EnvState*)h); }
 
 int g1_env_set_handover(void* h, int fences) {
   EnvState* E = (EnvState*)h;

@@ -324,7 +324,8 @@ __device__ __forceinline__ int finish_control_step(const PhysArgs& a, const Lane
 // worlds per wave: the policy's rollout of ra.ph.K control steps, or (policy false) K >= 1 control steps
 // on ra.ph.act.
 void launch_resident_kernel(const ResidentArgs& ra, bool policy, bool duo);
-// The rollout's function handles (occupancy report).
-const void* resident_kernel_fn(bool duo);
+// The instantiations' handles and block sizes (occupancy).
+const void* resident_kernel_fn(bool policy, bool duo);
+constexpr int resident_threads(bool duo) { return duo ? 2 * kPhysThreads : kPhysThreads; }
 
 }  // namespace g1k

@@ -12,7 +12,7 @@ namespace g1k {
 // nothing (its lanes would idle), and the contact phases run at the world's own contact count instead of
 // the larger of two. kPolicy: the actions come from the policy (K = H steps), else from ph.act.
 template <bool kDuo, bool kPolicy>
-__global__ void __launch_bounds__(kDuo ? 2 * kPhysThreads : kPhysThreads) k_resident(ResidentArgs ra) {
+__global__ void __launch_bounds__(resident_threads(kDuo)) k_resident(ResidentArgs ra) {
   constexpr int kW = kDuo ? 1 : 2;   // worlds per wave
   __shared__ __align__(16) WorldLds lds[2];
   __shared__ __align__(16) DuoLds duo[kDuo ? 2 : 1];
@@ -93,15 +93,16 @@ __global__ void __launch_bounds__(kDuo ? 2 * kPhysThreads : kPhysThreads) k_resi
 }
 
 void launch_resident_kernel(const ResidentArgs& ra, bool policy, bool duo) {
-  const dim3 grid((unsigned)(duo ? ra.ph.N : (ra.ph.N + 1) / 2)), block(duo ? 2 * kPhysThreads : kPhysThreads);
+  const dim3 grid((unsigned)(duo ? ra.ph.N : (ra.ph.N + 1) / 2)), block(resident_threads(duo));
   if (duo && policy) hipLaunchKernelGGL((k_resident<true, true>), grid, block, 0, 0, ra);
   else if (duo) hipLaunchKernelGGL((k_resident<true, false>), grid, block, 0, 0, ra);
   else if (policy) hipLaunchKernelGGL((k_resident<false, true>), grid, block, 0, 0, ra);
   else hipLaunchKernelGGL((k_resident<false, false>), grid, block, 0, 0, ra);
 }
 
-const void* resident_kernel_fn(bool duo) {
-  return duo ? (const void*)k_resident<true, true> : (const void*)k_resident<false, true>;
+const void* resident_kernel_fn(bool policy, bool duo) {
+  if (duo) return policy ? (const void*)k_resident<true, true> : (const void*)k_resident<true, false>;
+  return policy ? (const void*)k_resident<false, true> : (const void*)k_resident<false, false>;
 }
 
 }  // namespace g1k

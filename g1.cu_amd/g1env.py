@@ -55,6 +55,7 @@ SIGNATURES = {
     "g1_env_profile_read": (None, [_vp, _c.POINTER(_c.c_double)]),
     "g1_env_check": (_c.c_int, [_vp]),
     "g1_env_set_handover": (_c.c_int, [_vp, _c.c_int]),
+    "g1_env_launch_form": (_c.c_int, [_vp]),
     "g1_env_set_fused": (_c.c_int, [_vp, _c.c_int]),
     "g1_probe_qacc": (None, [_c.c_int, _vp, _vp, _vp, _c.c_int, _c.c_int, _c.c_int, _c.c_float, _vp, _vp]),
     "g1_probe_substep": (None, [_c.c_int, _vp, _vp, _vp, _c.c_int, _c.c_int, _c.c_float, _vp, _vp]),
@@ -174,6 +175,11 @@ class Env:
     def set_handover(self, fences):
         if lib.g1_env_set_handover(self.h, int(fences)) != 0:
             raise RuntimeError("hand-over mode unavailable on this placement")
+
+    def launch_form(self):
+        """How launches of this batch run: "queue", or resident waves: "duo" (a world on two waves) or "pair"
+        (two worlds per wave)."""
+        return ("queue", "duo", "pair")[lib.g1_env_launch_form(self.h)]
 
     def set_fused(self, on):
         """One persistent launch per rollout (True, the default) or per-step launches (False).

@@ -121,6 +121,12 @@ int g1_env_check(void* h);
  * g1_env_set_fused). Results are the same bit for bit. Returns 0, or -1 when the mode is unavailable. */
 int g1_env_set_handover(void* h, int fences);
 
+/* How a physics or one-launch rollout launch of this env runs, from its batch size and hand-over mode:
+ * 0 = the work queue, 1 = each world kept on two waves for the whole launch (batches that are resident
+ * at once in that form: up to 1024 worlds), 2 = two worlds kept per wave (up to 4096). The same results
+ * bit for bit. */
+int g1_env_launch_form(void* h);
+
 /* Rollout form: on = 1 (the default) runs g1_rollout as one persistent launch that interleaves the
  * policy of 16-world tiles with the physics work items, or, for batches that fit the chip at one or two
  * worlds per wave (up to 4096), keeps each wave's worlds for the whole launch (the same results bit for

@@ -1,7 +1,8 @@
 """Launches on batches that fit the chip (k_resident, up to 4096 worlds: one world on two waves up to 1024,
-then two per wave) against the work-queue form (k_rollout, k_physics), which the fenced
-hand-over keeps at every size: every output, the final state and the contact histogram bit for bit. The two forms share the physics, and the policy's sums run
-in the same order on the vector ALUs as on v_mfma_f32_16x16x4f32, so the tolerance is zero."""
+then two per wave) against the work-queue form (k_rollout, k_physics), which the fenced hand-over keeps at
+every size: every output, the final state and the contact histogram bit for bit. The two forms share the
+physics, and the policy's sums run in the same order on the vector ALUs as on v_mfma_f32_16x16x4f32, so the
+tolerance is zero. Each case asserts the form that it is about."""
 import numpy as np
 import pytest
 
@@ -17,17 +18,24 @@ def g1():
     return g1env
 
 
+def _form(N):
+    """The form of a batch at the default hand-over on the 256 CUs of an MI355X."""
+    return "duo" if N <= 1024 else "pair" if N <= 4096 else "queue"
+
+
 def _dev(x):
     import torch
     return torch.from_numpy(np.ascontiguousarray(x)).cuda()
 
 
-# the smallest batches; both sides of two waves per world and of two worlds per wave (odd counts); layers
-# of one to eight row blocks, ragged widths, one to three hidden layers; a horizon of zero
+# the smallest batches; both sides of two waves per world and of two worlds per wave (odd counts; 4097 worlds
+# take the queue with either hand-over); layers of one to eight row blocks, ragged widths, one to three hidden
+# layers; a horizon of zero
 @pytest.mark.parametrize("N,H,S,hidden,act,given", [
     (1, 3, 10, (256, 256), 0, False), (3, 2, 4, (17, 1), 1, True), (1023, 2, 5, (200, 72), 1, False),
     (1024, 2, 5, (256, 256), 0, True), (1025, 2, 5, (512, 512, 256), 1, True), (2047, 2, 4, (300,), 0, False),
-    (4095, 2, 4, (64, 513 - 1, 130), 0, False), (4096, 3, 3, (256, 256), 0, False), (40, 0, 10, (128, 65), 1, False),
+    (4095, 2, 4, (64, 513 - 1, 130), 0, False), (4096, 3, 3, (256, 256), 0, False), (4097, 2, 3, (256, 256), 0, False),
+    (4097, 2, 3, (300, 40), 1, False), (40, 0, 10, (128, 65), 1, False),
     (130, 12, 10, (256, 256), 0, False), (512, 3, 10, (256, 256), 0, True), (513, 3, 10, (256, 256), 0, True)])
 def test_resident_rollout_equals_work_queue(g1, N, H, S, hidden, act, given):
     import configs
@@ -45,6 +53,7 @@ def test_resident_rollout_equals_work_queue(g1, N, H, S, hidden, act, given):
         with g1.Env(N, substeps=S, pgs_iters=8, seed=9) as env:
             env.set_policy(hidden, act)
             env.set_handover(fences)
+            assert env.launch_form() == ("queue" if fences else _form(N))
             env.set_state(qp, qv, pa, steps)
             env.ncon_hist(enable=True)
             out = []
@@ -62,7 +71,7 @@ def test_resident_rollout_equals_work_queue(g1, N, H, S, hidden, act, given):
     assert H == 0 or (got[0][5] != 0).any()   # some world finished
 
 
-@pytest.mark.parametrize("N,S", [(1, 10), (33, 1), (512, 10), (513, 10), (1024, 5), (1025, 4), (4095, 3)])
+@pytest.mark.parametrize("N,S", [(1, 10), (33, 1), (512, 10), (513, 10), (1024, 5), (1025, 4), (4095, 3), (4096, 2)])
 def test_resident_control_steps_equal_work_queue(g1, N, S):
     """Host steps (observation, reward, done; a finished world restarts) and zero-action physics: the two forms'
     outputs and states bit for bit."""
@@ -76,6 +85,7 @@ def test_resident_control_steps_equal_work_queue(g1, N, S):
     for fences in (0, 1):
         with g1.Env(N, substeps=S, pgs_iters=8, seed=4) as env:
             env.set_handover(fences)
+            assert env.launch_form() == ("queue" if fences else _form(N))
             env.set_state(qp, qv, pa, steps)
             env.ncon_hist(enable=True)
             out = [x for a in acts for x in env.step(a)]
