@@ -71,6 +71,49 @@ def test_resident_rollout_equals_work_queue(g1, N, H, S, hidden, act, given):
     assert H == 0 or (got[0][5] != 0).any()   # some world finished
 
 
+@pytest.mark.parametrize("hidden,act", [((256, 256), 0), ((256, 256), 1), ((512, 512, 256), 1)])
+@pytest.mark.parametrize("N", [64, 1030])
+@pytest.mark.parametrize("scale", ["wide", "subnormal", "huge"])
+def test_policy_sums_equal_mfma_over_the_range_of_fp32(g1, scale, N, hidden, act):
+    """The resident policy's fma chains against the MFMA tiles' sums where their order and rounding show most:
+    weights spread over 2^-40 .. 2^40; weights whose products and sums are subnormal; weights whose sums overflow.
+    Every output of one control step and the bootstrap value bit for bit (NaN against NaN)."""
+    import configs
+    import torch
+    rng = np.random.default_rng(5)
+    qp, qv, pa, steps = configs.reset_states(rng, N)
+    qv = rng.normal(0, 0.3, qv.shape).astype(np.float32)
+    W = configs.policy_init(rng, hidden=hidden)
+    n = W.size - 29   # the log standard deviations stay
+    if scale == "wide":
+        W[:n] *= np.exp2(rng.integers(-40, 41, n)).astype(np.float32)
+    elif scale == "subnormal":
+        n = 100 * hidden[0]   # the first layer: subnormal activations through the others
+        W[:n] *= np.exp2(rng.integers(-142, -127, n)).astype(np.float32)
+    else:
+        W[:n] *= np.exp2(rng.integers(40, 127, n)).astype(np.float32)
+    W, mean, var = _dev(W), _dev(np.zeros(100, np.float32)), _dev(np.ones(100, np.float32))
+    got = []
+    for fences in (0, 1):
+        with g1.Env(N, substeps=1, pgs_iters=8, seed=9) as env:
+            env.set_policy(hidden, act)
+            env.set_handover(fences)
+            assert env.launch_form() == ("queue" if fences else _form(N))
+            env.set_state(qp, qv, pa, steps)
+            tr = g1.Trajectory(1, N)
+            tr.run(env, W, mean, var)
+            torch.cuda.synchronize()
+            got.append(tr.numpy())
+            assert env.check() == 0
+    for f in g1.Trajectory.FIELDS:
+        a, b = (x[f] for x in got)
+        assert np.array_equal(np.where(np.isnan(a), 0, a.view(np.uint32)), np.where(np.isnan(b), 0, b.view(np.uint32))), f
+        assert np.array_equal(np.isnan(a), np.isnan(b)), f
+    V = got[0]["V"]
+    if scale == "subnormal":
+        assert (np.abs(V) < np.finfo(np.float32).tiny).all() and (V != 0).mean() > 0.5
+
+
 @pytest.mark.parametrize("N,S", [(1, 10), (33, 1), (512, 10), (513, 10), (1024, 5), (1025, 4), (4095, 3), (4096, 2)])
 def test_resident_control_steps_equal_work_queue(g1, N, S):
     """Host steps (observation, reward, done; a finished world restarts) and zero-action physics: the two forms'

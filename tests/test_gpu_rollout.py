@@ -2,10 +2,14 @@
 the CPU oracle on identical states and pre-generated noise.
 
 Teacher forcing: every control step starts the oracle from the GPU's own state before that step
-(g1_env_get_state). The policy runs on MFMA and its outputs are held to the per-step bound (A/LP/V
-within 1e-5, O bitwise). The physics of a step is driven by the GPU's own actions and compared bit
+(g1_env_get_state). The policy runs on MFMA tiles or, on resident waves, as matrix-vector products; its
+outputs are held to the per-step bound (A/LP/V within 1e-5, O bitwise). The physics of a step is driven by the GPU's own actions and compared bit
 for bit with the oracle in the kernel's summation association: qpos, qvel, reward, done, step
 counters and reset states.
+
+A batch of up to 4096 worlds runs on resident waves (k_resident: "duo" up to 1024 worlds, then
+"pair"), a larger one, or any with the fenced hand-over, on the work queue (k_rollout, k_physics);
+tests about one of the forms assert which one they run.
 """
 import os
 
@@ -175,14 +179,17 @@ def test_rollout_teacher_forced_config4_slice(g1, orc):
     _assert_rows(rows)
 
 
+@pytest.mark.parametrize("form", ["queue", "duo"])
 @pytest.mark.parametrize("hidden,act", [((48, 32), 1), ((80, 144), 0), ((100, 60), 0), ((256, 17), 1),
                                         ((512, 512, 256), 1), ((300,), 0), ((64, 48, 32), 1), ((512, 70), 0)])
-def test_rollout_teacher_forced_one_launch_shapes(g1, orc, hidden, act):
-    """The one-launch rollout's policy tiles on shapes other than 256-256: two layers of at most 256
-    run on the register-resident tile at 256-256 with zero padding (widths that are and are not
-    multiples of 16, ELU and tanh); one to three layers of up to 512 on the wide tile (activations
-    staged in global memory, output tiles padded to multiples of 64 rows), config 4's 512-512-256
-    ELU among them. N=512, 4 control steps against the oracle."""
+def test_rollout_teacher_forced_one_launch_shapes(g1, orc, hidden, act, form):
+    """The one-launch rollout's policy on shapes other than 256-256. In the work queue (the fenced
+    hand-over): two layers of at most 256 on the register-resident tile at 256-256 with zero padding
+    (widths that are and are not multiples of 16, ELU and tanh); one to three layers of up to 512 on
+    the wide tile (activations staged in global memory, output tiles padded to multiples of 64
+    rows), config 4's 512-512-256 ELU among them. On resident waves (the default at this size): the
+    same shapes as matrix-vector products over each world's rows. N=512, 4 control steps against
+    the oracle."""
     import configs
     N, H = 512, 4
     rng = np.random.default_rng(61)
@@ -192,6 +199,8 @@ def test_rollout_teacher_forced_one_launch_shapes(g1, orc, hidden, act):
     var = rng.uniform(0.5, 2.0, 100).astype(np.float32)
     with g1.Env(N, substeps=10, pgs_iters=8, seed=1) as env:
         env.set_policy(hidden, act)
+        env.set_handover(int(form == "queue"))
+        assert env.launch_form() == form
         assert env.policy_params() == W.size
         assert env.set_fused(True)          # the shape runs in the one-launch form
         env.set_state(qp, qv, pa, steps)
@@ -228,16 +237,20 @@ def test_one_launch_rollout_equals_step_by_step(g1):
     assert one["D"].sum() > 0
 
 
-@pytest.mark.parametrize("fences,fused", [(0, True), (1, True), (0, False), (1, False)])
-def test_rollout_matches_oracle_free_run(g1, orc, fences, fused):
-    """A short rollout (N=96, H=3) with no teacher forcing: every output equals the oracle's own
-    rollout within the per-step bound, in both rollout forms (one persistent launch, or policy and
-    physics launches per control step), through the L2 state hand-over (fences=0) and through the
-    agent-scope fence hand-over that the work queue falls back to off the round-robin placement."""
-    N, H = 96, 3
+@pytest.mark.parametrize("N,fences,fused,form", [
+    (96, 0, True, "duo"), (96, 1, True, "queue"), (96, 0, False, "duo"), (96, 1, False, "queue"),
+    (1027, 0, True, "pair"), (4097, 0, True, "queue"), (4097, 0, False, "queue")])
+def test_rollout_matches_oracle_free_run(g1, orc, N, fences, fused, form):
+    """A short rollout (H=3) with no teacher forcing: every output equals the oracle's own rollout
+    within the per-step bound, in both rollout forms (one launch, or policy and physics launches per
+    control step) and every form of a launch: resident waves, the work queue with the L2 state
+    hand-over (4097 worlds, fences=0), and the work queue with the agent-scope fence hand-over that
+    it falls back to off the round-robin placement."""
+    H = 3
     qp, qv, pa, steps, W, mean, var, an, rn = _setup(N, H, 11)
     with g1.Env(N, substeps=10, pgs_iters=8, seed=1) as env:
         env.set_handover(fences)
+        assert env.launch_form() == form
         assert env.set_fused(fused) == fused
         env.set_state(qp, qv, pa, steps)
         out = _rollout(g1, env, W, mean, var, H, an, rn)
@@ -401,13 +414,14 @@ def test_host_step_matches_oracle(g1, orc):
     assert np.array_equal(obs1[live], orc.obs(oq, ov, opa)[live])
 
 
+@pytest.mark.parametrize("form", ["queue", "duo"])
 @pytest.mark.parametrize("path", ["host_step", "rollout"])
-def test_velocity_guard_nan_inf_and_clamp(g1, orc, path):
+def test_velocity_guard_nan_inf_and_clamp(g1, orc, path, form):
     """The env's velocity guard (src/g1_env.cu:154-160: a non-finite velocity becomes 0, then the
     clamp to +-50) on the GPU, against the oracle bit for bit: worlds start with NaN, +-inf and
     +-1e4 velocities on base and hinge dofs (g1_env_set_state) beside ordinary ones and take one
-    control step through the host-step path (k_physics) or a one-step rollout (k_rollout). The
-    reference's comparison clamps let NaN through everywhere else, as the kernels do: a NaN hinge
+    control step through the host-step path or a one-step rollout, each on the work queue (k_physics,
+    k_rollout; the fenced hand-over) and on resident waves (k_resident). The reference's comparison clamps let NaN through everywhere else, as the kernels do: a NaN hinge
     velocity makes that step's reward NaN and, in the rollout, the world's observation and action
     NaN; the guard leaves every velocity finite and within +-50."""
     import configs
@@ -424,6 +438,8 @@ def test_velocity_guard_nan_inf_and_clamp(g1, orc, path):
     W = configs.policy_init(rng)
     mean, var = np.zeros(100, np.float32), np.ones(100, np.float32)
     with g1.Env(N, substeps=10, pgs_iters=8, seed=4) as env:
+        env.set_handover(int(form == "queue"))
+        assert env.launch_form() == form
         env.set_state(qp, qv, pa, steps)
         if path == "host_step":
             _, rew, done = env.step(act)
@@ -457,37 +473,43 @@ def test_velocity_guard_nan_inf_and_clamp(g1, orc, path):
 def test_work_queue_matches_small_launch(g1):
     """The physics work queue at scale: a rollout over 8193 worlds (many work items per wave, state
     handed between waves, an odd last pair) gives each of its first 97 worlds bit for bit the
-    trajectory those worlds get in a 97-world launch (world 96 then has no partner); the same with
-    the fence hand-over."""
+    trajectory those worlds get in a 97-world launch of the queue (the fenced hand-over; world 96
+    then has no partner) and on resident waves; the same 8193 worlds with the fence hand-over."""
     H, N, n = 3, 8193, 97
     qp, qv, pa, steps, W, mean, var, an, rn = _setup(N, H, 21)
     runs = []
-    for m, fences in ((N, 0), (n, 0), (N, 1)):
+    for m, fences, form in ((N, 0, "queue"), (n, 1, "queue"), (N, 1, "queue"), (n, 0, "duo")):
         with g1.Env(m, substeps=10, pgs_iters=8, seed=1) as env:
             env.set_handover(fences)
+            assert env.launch_form() == form
             env.set_state(qp[:m], qv[:m], pa[:m], steps[:m])
             out = _rollout(g1, env, W, mean, var, H, np.ascontiguousarray(an[:, :m]), np.ascontiguousarray(rn[:, :m]))
             runs.append((out, env.get_state()))
-    (big, big_state), (small, small_state), (fen, fen_state) = runs
+    (big, big_state), (small, small_state), (fen, fen_state), (res, res_state) = runs
     for f in g1.Trajectory.FIELDS:
         k = (slice(None), slice(0, n)) if big[f].ndim >= 2 else slice(0, n)
         assert np.array_equal(big[f][k], small[f]), f
         assert np.array_equal(big[f], fen[f]), f
-    for b, s, e in zip(big_state, small_state, fen_state):
-        assert np.array_equal(b[:n], s) and np.array_equal(b, e)
+        assert np.array_equal(big[f][k], res[f]), f
+    for b, s, e, r in zip(big_state, small_state, fen_state, res_state):
+        assert np.array_equal(b[:n], s) and np.array_equal(b, e) and np.array_equal(b[:n], r)
     assert not np.array_equal(big_state[0], qp)   # the worlds moved
 
 
+@pytest.mark.parametrize("form", ["queue", "duo"])
 @pytest.mark.parametrize("n", [1, 2, 3])
-def test_rollout_of_one_to_three_worlds(g1, n):
-    """Ragged smallest sizes: a rollout of n = 1, 2, 3 worlds (one or two pairs, an odd last pair;
-    31 of the 32 work queues empty, their blocks drain the one queue of their XCD or exit) gives
-    those worlds bit for bit the trajectory they get as the first n worlds of a 64-world launch."""
+def test_rollout_of_one_to_three_worlds(g1, n, form):
+    """Ragged smallest sizes: a rollout of n = 1, 2, 3 worlds gives those worlds bit for bit the
+    trajectory they get as the first n worlds of a 64-world launch, on the work queue (the fenced
+    hand-over: one or two pairs, an odd last pair; 30 or 31 of the 32 queues empty, their blocks
+    drain the other queues of their XCD or exit) and on resident waves (one to three blocks)."""
     H, N = 4, 64
     qp, qv, pa, steps, W, mean, var, an, rn = _setup(N, H, 31)
     runs = []
     for m in (N, n):
         with g1.Env(m, substeps=10, pgs_iters=8, seed=5) as env:
+            env.set_handover(int(form == "queue"))
+            assert env.launch_form() == form
             env.set_state(qp[:m], qv[:m], pa[:m], steps[:m])
             out = _rollout(g1, env, W, mean, var, H, np.ascontiguousarray(an[:, :m]), np.ascontiguousarray(rn[:, :m]))
             runs.append((out, env.get_state()))
@@ -499,16 +521,22 @@ def test_rollout_of_one_to_three_worlds(g1, n):
         assert np.array_equal(b[:n], s)
 
 
-@pytest.mark.parametrize("N,S,K", [(301, 5, 3), (301, 10, 200)])
-def test_work_queue_split_control_steps(g1, N, S, K):
+@pytest.mark.parametrize("N,S,K,fences,form", [
+    (301, 5, 3, 1, "queue"), (301, 10, 200, 1, "queue"), (4099, 5, 3, 0, "queue"), (4099, 10, 9, 0, "queue"),
+    (301, 5, 3, 0, "duo"), (301, 10, 200, 0, "duo"), (1301, 10, 20, 0, "pair")])
+def test_work_queue_split_control_steps(g1, N, S, K, fences, form):
     """K control steps in one physics launch equal K one-step launches bit for bit: S = 5 (items of
-    3 and 2 substeps, an odd world count), and S = 10 with K = 200 (at least 8 pair-steps per wave,
-    so items of 6 and 4 substeps, against 3, 3, 2, 2 for the one-step launches)."""
+    3 and 2 substeps, an odd world count), and S = 10 with K = 200 or, at 2050 pairs on 2048 waves,
+    K = 9 (at least 8 pair-steps per wave, so items of 6 and 4 substeps, against 3, 3, 2, 2 for the
+    one-step launches), with both hand-overs of the queue; and on resident waves, which keep their
+    worlds from step to step in the one launch and take them from memory in each of the others."""
     import configs
     qp, qv, pa, steps = configs.reset_states(np.random.default_rng(5), N)
     states = []
     for split in (False, True):
         with g1.Env(N, substeps=S, pgs_iters=8, seed=2) as env:
+            env.set_handover(fences)
+            assert env.launch_form() == form
             env.set_state(qp, qv, pa, steps)
             for _ in range(K if split else 1):
                 env.bench_phys(1 if split else K)
@@ -518,11 +546,15 @@ def test_work_queue_split_control_steps(g1, N, S, K):
     assert not np.array_equal(states[0][0], qp)
 
 
-def test_host_step_five_substeps_matches_oracle(g1, orc):
-    """g1_env_step with S = 5 (a control step split into work items of 3 and 2 substeps, its reward
-    sums carried between items) against the oracle's control step."""
-    N, S = 129, 5
+@pytest.mark.parametrize("N,fences,form", [(129, 1, "queue"), (4097, 0, "queue"), (129, 0, "duo")])
+def test_host_step_five_substeps_matches_oracle(g1, orc, N, fences, form):
+    """g1_env_step with S = 5 against the oracle's control step: on the work queue with both
+    hand-overs (the control step split into work items of 3 and 2 substeps, its reward sums carried
+    between items) and on resident waves."""
+    S = 5
     with g1.Env(N, substeps=S, pgs_iters=8, seed=3) as env:
+        env.set_handover(fences)
+        assert env.launch_form() == form
         env.reset()
         qp, qv, pa, st = env.get_state()
         act = np.random.default_rng(6).normal(0, 0.3, (N, 29)).astype(np.float32)
@@ -532,6 +564,40 @@ def test_host_step_five_substeps_matches_oracle(g1, orc):
     live = dd == 0
     assert np.array_equal(done, dd) and np.array_equal(rew, rr)
     assert np.array_equal(obs1[live], orc.obs(oq, ov, opa)[live])
+
+
+@pytest.mark.parametrize("fences", [0, 1])
+@pytest.mark.parametrize("N", [4096, 4097, 8191])
+def test_host_step_of_large_batches_matches_oracle(g1, orc, N, fences):
+    """g1_env_reset and g1_env_step on both sides of the size up to which the kernels write the
+    outputs straight into pinned memory (4096 worlds; past it they go through device memory in four
+    chunks of worlds, the last one ragged at 4097 and 8191): reset's observations are those of the
+    state it left; two control steps in a row give rewards, done flags and the observations of every
+    world, finished ones included (reset by the library's noise stream, replayed here), bit for bit
+    as the oracle."""
+    import philox_np
+    rng = np.random.default_rng(N)
+    with g1.Env(N, substeps=10, pgs_iters=8, seed=3) as env:
+        env.set_handover(fences)
+        assert env.launch_form() == ("queue" if fences or N > 4096 else "pair")
+        obs = env.reset()
+        qp, qv, pa, st = env.get_state()
+        assert np.array_equal(obs, orc.obs(qp, qv, pa))
+        st[::11] = 998   # time-outs at the second step, all over the chunks
+        st[-1] = 999     # and one at the first step in the last world
+        env.set_state(qp, qv, pa, st)
+        for k in range(2):
+            act = rng.normal(0, 0.3, (N, 29)).astype(np.float32)
+            obs, rew, done = env.step(act)
+            # the reset drew with counter 0, so step k draws with counter 1 + k
+            noise = philox_np.uniform_pm1(3, np.arange(N), 1 + k, philox_np.STREAM_RESET).astype(np.float32)
+            rr, dd = orc.env_advance(qp, qv, pa, st, act, noise, threads=NTHREADS)
+            assert np.array_equal(done, dd) and np.array_equal(rew, rr), k
+            assert np.array_equal(obs, orc.obs(qp, qv, pa)), k
+            assert dd.any()
+        for a, b in zip(env.get_state(), (qp, qv, pa, st)):
+            assert np.array_equal(a, b)
+        assert env.check() == 0
 
 
 def test_reference_trained_policy_walks(g1):

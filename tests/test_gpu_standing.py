@@ -45,14 +45,15 @@ def test_stability_gate(g1):
     assert not done_any.any()
 
 
-def test_bench_phys_matches_oracle_standing(g1, orc):
+@pytest.mark.parametrize("N,form", [(1024, "duo"), (1026, "pair"), (4099, "queue")])
+def test_bench_phys_matches_oracle_standing(g1, orc, N, form):
     """g1_env_bench_phys (zero action, reward/termination/auto-reset included) against the oracle's
     zero-action control step, teacher-forced from the GPU's state before each of 4 control steps:
     qpos, qvel, step counters and previous actions bit for bit (the oracle in the kernel's
-    summation association)."""
-    N = 1024
+    summation association), in each form of a launch at the default hand-over."""
     worst = []
     with g1.Env(N, substeps=10, pgs_iters=8, seed=5) as env:
+        assert env.launch_form() == form
         env.reset()
         for t in range(4):
             pre = env.get_state()

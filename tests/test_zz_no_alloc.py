@@ -6,7 +6,8 @@ call). Each no-alloc call runs on a fresh env and leaves the env's device memory
 it (g1_env_device_bytes), while g1_rollout_ex on a fresh env grows it by its packed policy. A policy
 wider than two layers of 256 runs the no-alloc call in the per-step form (the one-launch form's wide
 tile needs activation buffers the library allocates), so its g1_rollout_ex comparison takes the
-per-step form too."""
+per-step form too. Both on resident waves (the default at these sizes) and on the work queue (the
+fenced hand-over)."""
 import numpy as np
 import pytest
 
@@ -33,13 +34,15 @@ def _case(N, H, hidden, seed):
     return (qp, qv, pa, st), (W, mean, var, an, rn)
 
 
-def _run(g1, state, inputs, N, H, hidden, act, noalloc):
+def _run(g1, state, inputs, N, H, hidden, act, form, noalloc):
     """One rollout on a fresh env; returns the outputs, the final state and the env's device bytes
     before and after the call."""
     import torch
     dev = [torch.from_numpy(np.ascontiguousarray(x)).cuda() for x in inputs]
     with g1.Env(N, substeps=10, pgs_iters=8, seed=3) as env:
         env.set_policy(hidden, act)
+        env.set_handover(int(form == "queue"))
+        assert env.launch_form() == form
         narrow = len(hidden) == 2 and max(hidden) <= 256
         env.set_fused(narrow)   # the form g1_rollout_noalloc takes for this shape
         env.set_state(*state)
@@ -56,12 +59,13 @@ def _run(g1, state, inputs, N, H, hidden, act, noalloc):
         return traj.numpy(), env.get_state(), (before, after)
 
 
-def test_noalloc_rollout_matches_allocating_rollout(g1):
+@pytest.mark.parametrize("form", ["queue", "duo"])
+def test_noalloc_rollout_matches_allocating_rollout(g1, form):
     cases = [(96, 3, (512, 512, 256), 1, 71), (40, 2, (256, 256), 0, 72)]   # second: smaller everything
     for N, H, hidden, act, seed in cases:
         state, inputs = _case(N, H, hidden, seed)
-        ref, ref_state, (b0, b1) = _run(g1, state, inputs, N, H, hidden, act, noalloc=False)
-        got, got_state, (n0, n1) = _run(g1, state, inputs, N, H, hidden, act, noalloc=True)
+        ref, ref_state, (b0, b1) = _run(g1, state, inputs, N, H, hidden, act, form, noalloc=False)
+        got, got_state, (n0, n1) = _run(g1, state, inputs, N, H, hidden, act, form, noalloc=True)
         assert b1 > b0, (N, b0, b1)          # the allocating form packed into a buffer it allocated
         assert n1 == n0 == b0, (N, n0, n1)   # the no-alloc form allocated nothing
         for f in g1.Trajectory.FIELDS:
