@@ -13,6 +13,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 #include "../../include/g1env.h"
@@ -978,6 +979,30 @@ static void scratch_setup() {
   scratch_addr[dev] = (float*)p;
 }
 
+// The worlds that k_resident holds on a GPU at once: one world per block on two waves (duo), two on one wave
+// (pair); both instantiations of a form have to be resident. Facts of the kernels and the GPU, asked for once
+// per device (four occupancy queries took 0.15 ms of an env's creation).
+struct ResidentLimits {
+  std::once_flag once;
+  int duo, pair;
+};
+static const ResidentLimits& resident_limits(int dev, int cus) {
+  static ResidentLimits table[kMaxDevices];   // (scratch_setup checks the index)
+  ResidentLimits& r = table[dev];
+  std::call_once(r.once, [&] {
+    auto blocks = [&](bool duo) {
+      int n[2];
+      for (int policy = 0; policy < 2; ++policy)
+        HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n[policy], resident_kernel_fn(policy, duo),
+                                                              resident_threads(duo), 0));
+      return cus * std::min(n[0], n[1]);
+    };
+    r.duo = blocks(true);
+    r.pair = 2 * blocks(false);
+  });
+  return r;
+}
+
 extern "C" {
 
 int g1_env_obs_dim(void) { return kObs; }
@@ -1026,16 +1051,9 @@ void* g1_env_create(int N, int substeps, int pgs_iters, unsigned long seed) {
     if (cap < kQueues) cap = kQueues;
     const int need = (npairs + kQueues - 1) / kQueues * kQueues;
     E->pgrid = need < cap ? need : cap;
-    // one world per block on two waves, two on one wave; both instantiations of a form have to be resident
-    auto resident_blocks = [&](bool duo) {
-      int n[2];
-      for (int policy = 0; policy < 2; ++policy)
-        HIPCHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&n[policy], resident_kernel_fn(policy, duo),
-                                                              resident_threads(duo), 0));
-      return cus * std::min(n[0], n[1]);
-    };
-    E->duo_worlds = resident_blocks(true);
-    E->pair_worlds = 2 * resident_blocks(false);
+    const ResidentLimits& rl = resident_limits(dev, cus);
+    E->duo_worlds = rl.duo;
+    E->pair_worlds = rl.pair;
     // placement of the blocks on the XCDs: round-robin lets each queue hand over state in one L2
     int* dx = nullptr;
     HIPCHECK(hipMalloc(&dx, (size_t)E->pgrid * sizeof(int)));
