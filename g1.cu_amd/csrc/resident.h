@@ -74,9 +74,12 @@ __device__ __forceinline__ void net_inputs(const float* x, float4 (&xu)[V]) {
 // whose 32 rows take half a wave: lanes 0..31 serve one world and lanes 32..63 the other (x is the
 // lane's own world's).
 static_assert(kNetBuf >= kMaxHidden + 4, "a unit past the inputs is inside the buffer");
-template <int V, int R, int kAhead, bool kHead>
+template <int V, int R, bool kHead>
 __device__ __forceinline__ void net_pass(const float4* W, const float* bias, int nQ, int T0, const float* x, int lane,
                                          float (&acc)[V][R]) {
+  // four quads ahead in the head; one in the hidden layers, where two would take the kernel to the register limit
+  // of two waves per SIMD, at which the physics' schedule is slower (32 steps of 1024 worlds 3.39 -> 3.55 ms)
+  constexpr int kAhead = kHead ? 4 : 1;
   const int j = lane & 15, tt = kHead ? (lane >> 4) & 1 : lane >> 4;
   const char* base[R];
 #pragma unroll
@@ -113,12 +116,10 @@ __device__ __forceinline__ void net_pass(const float4* W, const float* bias, int
 #pragma unroll
     for (int v = 0; v < V; ++v) xc[v] = xn[v];
   };
-  static_assert(kAhead == 1 || kAhead == 2 || kAhead == 4, "nQ is 7 (layer 0) or a multiple of 4");
 #pragma unroll 1
-  for (int q = 0; q < nQ; q += kAhead) {
+  for (int q = 0; q < nQ; q += kAhead) {   // nQ is 7 (layer 0) or a multiple of 4 (all others, the head's too)
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) {
-      if (i > 0 && !kHead && q + i >= nQ) break;
       if (q + i + kAhead >= nQ) {   // past the end: the last quad again
 #pragma unroll
         for (int r = 0; r < R; ++r) base[r] -= 1024;
@@ -138,11 +139,8 @@ __device__ __forceinline__ void net_pass(const float4* W, const float* bias, int
 template <int kW, int R>
 __device__ __forceinline__ void net_rows(const float4* W, const float* bias, int nQ, int T0, const float* x, float* out,
                                          int act, int lane) {
-  // one quad's weights ahead: two take the kernel to the register limit of two waves per SIMD, where the
-  // physics' schedule is slower (32 steps of 1024 worlds 3.39 -> 3.55 ms)
-  constexpr int kAhead = 1;
   float acc[kW][R];
-  net_pass<kW, R, kAhead, false>(W, bias, nQ, T0, x, lane, acc);
+  net_pass<kW, R, false>(W, bias, nQ, T0, x, lane, acc);
 #pragma unroll
   for (int v = 0; v < kW; ++v)
 #pragma unroll
@@ -234,7 +232,7 @@ __device__ __forceinline__ float wave_policy(const TileArgs& a, const LaneState&
   if (kDuo && role != 0) return 0.f;
   // ---- head: lane (v, 16 ht + j) has row i = 16 ht + j of world v (mu 0..28, value 29)
   float hd[1][1];
-  net_pass<1, 1, 4, true>(W + T.woff[T.nl] / 4, a.Wt + T.boff[T.nl], T.nQ[T.nl], 0, mine + (T.nl & 1) * kNetBuf, lane, hd);
+  net_pass<1, 1, true>(W + T.woff[T.nl] / 4, a.Wt + T.boff[T.nl], T.nQ[T.nl], 0, mine + (T.nl & 1) * kNetBuf, lane, hd);
   const int i = l;
   if (i == kAct && wvalid) {
     if (t == a.H) a.Vlast[w] = hd[0][0];
