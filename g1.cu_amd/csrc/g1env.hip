@@ -1,11 +1,13 @@
 // g1env.hip -- MI355X (gfx950) implementation of g1.cu's batched G1 environment and fused PPO
 // rollout behind the reference's libg1env.so C ABI (reference: src/g1_env.cu:361-476).
 //
-// Rollout structure: g1_rollout enqueues, on the null stream and without any host sync,
-//   pack(W) -> [policy(t) -> physics(t)] for t < H -> policy(H) (bootstrap value)
-// policy(t): obs -> frozen normalisation -> MLP on fp32 MFMA over 32-world tiles -> sampling;
-// physics(t): S substeps of FK -> PD -> world_qacc -> Euler on 32-lane world groups, then reward,
-// termination and auto-reset. Trajectory tensors O/A/LP/V/R/D/Vlast are caller-owned device
+// Rollout structure: g1_rollout enqueues, on the null stream and without any host sync, pack(W) and one
+// launch that runs policy(t) -> physics(t) for t < H and policy(H) (the bootstrap value): k_resident for
+// batches that fit the chip (resident.h), else k_rollout (queue.h). After g1_env_set_fused(h, 0), and for
+// wide policies in g1_rollout_noalloc, policy (k_policy) and physics are launches of their own per step.
+// policy(t): obs -> frozen normalisation -> MLP (fp32 MFMA tiles of 16 or 32 worlds, or matrix-vector
+// products) -> sampling; physics(t): S substeps of FK -> PD -> world_qacc -> Euler on 32-lane world groups,
+// then reward, termination and auto-reset. Trajectory tensors O/A/LP/V/R/D/Vlast are caller-owned device
 // buffers written in place, exactly as the reference's k_rollout does (src/g1_env.cu:278-338).
 #include <hip/hip_runtime.h>
 
@@ -766,12 +768,13 @@ static void chunk_schedule(PhysArgs& a, int pgrid, bool one_launch = false) {
 
 // The form of a launch: one world on two waves of k_resident while all of them are resident at once (1024
 // worlds), two worlds per wave while that holds for those (4096), and the work queue past that, where a
-// second round of waves would start when the first ends and the queue spreads the work evenly. Measured,
-// ms per rollout of the 256-256 policy with one world on two waves, one per wave, two per wave, and the
-// queue: 16 steps of 256 worlds 1.50, 1.63, 1.83, 2.55; 768 1.64, 1.75, 1.96, -; 32 steps of 1024 3.22,
-// 3.34, 3.85, 5.42; 1536 -, 3.86, 3.87, 5.48; 2048 -, 3.99, 3.81, 5.51; 4096 -, -, 4.46, 6.02 (8192 on the
-// queue 7.6). Five control steps on given actions, us, of 1024 standing worlds: 796, 837, 850, 930. An
-// env set to the fenced hand-over keeps the queue, which that mode is about.
+// second round of waves would start when the first ends and the queue spreads the work evenly. Measured on
+// both sides of the lines with one world on two waves, two worlds per wave and the queue (each forced): ms
+// per rollout of the 256-256 policy, 16 steps of 256 worlds 1.52, 1.81, 2.42; 768 1.76, 2.00, 2.58; 32 steps
+// of 1024 3.52, 3.83, 5.14; 1536 6.20, 3.78, 5.19; 2048 8.21, 4.23, 5.22; 4096 -, 4.56, 5.77; 4608 -, 7.56,
+// 5.90; 8192 -, 8.61, 7.54; 512-512-256 policy, 4 steps of 512 0.58, 0.71, 1.22. Five control steps of standing
+// worlds on given actions, us: 1 world 743, 796, 816; 1024 822, 858, 879; 4096 -, 983, 1020; 8192 -, 1921,
+// 1904. An env set to the fenced hand-over keeps the queue, which that mode is about.
 enum class Form { kQueue, kDuo, kPair };   // (values: g1_env_launch_form)
 static Form launch_form(const EnvState* E) {
   if (E->fences) return Form::kQueue;
@@ -1107,8 +1110,9 @@ void g1_env_destroy(void* h) {
 
 // Whether the host-step path's kernels write their outputs straight into pinned host memory: batches that
 // fit the chip at once, whose step is a matter of tens of microseconds of copies and synchronisations
-// (us per step, through device memory and directly: 1 world 149, 122; 1024 282, 181; 4096 330, 269). Of
-// larger outputs the host copies one part while the next is transferred (8192 worlds 479; directly 513).
+// (us per step, through device memory and directly: 1 world 136, 114; 1024 237, 180; 4096 309, 284). Of
+// larger outputs the host copies one part while the next is transferred (8192 worlds 507; directly 526; just
+// past the line, 4097 worlds, direct outputs would still be ahead, 331 against 300).
 static bool direct_outputs(const EnvState* E) { return E->N <= E->pair_worlds; }
 
 // The observations, and with rew the rewards and done flags, from the device's [obs | reward | done] to

@@ -7,15 +7,16 @@
 // saves: one wave computes the tile in 43 us while the tile's other seven waves wait for it, each step
 // of all 16 worlds starts when the slowest of the eight pairs has finished the last one, and state,
 // actions and flags cross the L2 between the waves. Here nothing is waited for but the world's own work.
-// Bound by one wave's instruction issue (about one per four cycles): 8 to 9 us per substep, and 10 to 13 us
-// for the rest of a control step, most of it the 256-256 policy (its weights' way from the L2). Up to 1024
-// worlds a second wave, on a SIMD that would stand idle or carry one wave, takes part of each substep's
-// physics (world_qacc<true>) and half of the policy's rows (16 steps of 256 worlds 1.51 -> 1.47 ms by the
-// latter; 4 steps of 512 with the 512-512-256 policy 0.63 -> 0.57). Rollouts against the queue: 16 steps of
-// 256 worlds 2.55 -> 1.47 ms, 32 steps of 1024 5.42 -> 3.18, 2048 5.51 -> 3.75, 4096 6.02 -> 4.4; 512-512-256
-// policy, 4 steps of 512 worlds 1.26 -> 0.57, 8 steps of 4096 2.83 -> 1.81. Control steps on given actions (the host step, g1_env_bench_phys): one
-// world, a step 149 -> 106 us (of it 27 the outputs' way to the host), 5 steps of 1024 standing worlds 930
-// -> 796.
+// Bound by one wave's instruction stream: with 256 worlds on two waves each the VALU is busy 17% of the time,
+// and a wave that is not at a barrier issues in about 70% of its cycles and waits for LDS and memory in most
+// of the others. A substep takes 8 us (19.4k cycles; standing worlds 35.5k), the policy 10.5 us per control
+// step (25k cycles, 15.6k of them the hidden layers of 256-256: their weights' way from the L2), with two
+// worlds per wave 10 and 15.5. Up to 1024 worlds a second wave, on a SIMD that would stand idle or carry one
+// wave, takes part of each substep's physics (world_qacc<true>) and half of the policy's rows (16 steps of
+// 256 worlds 1.51 -> 1.47 ms by the latter; 4 steps of 512 with the 512-512-256 policy 0.63 -> 0.57). Rollouts
+// against the queue: 16 steps of 256 worlds 2.55 -> 1.48 ms, 32 steps of 1024 5.45 -> 3.17, 24 steps of 3001 (5
+// substeps) 2.79 -> 1.72; 512-512-256 policy, 4 steps of 512 worlds 1.26 -> 0.57. One world's host step 149 ->
+// 104 us; the other sizes and the control steps on given actions: launch_form.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -34,9 +35,9 @@ struct ResidentArgs {
 // (400 KB per pass for 256-256), not by arithmetic, and an MFMA would leave 14 of its 16 columns idle.
 // Each lane computes whole rows (neurons) of a layer: in a pass over the tiles T0 .. T0 + 4 R - 1 lane
 // 16 tt + j takes row j of the tiles T0 + 4 r + tt, r < R. v_mfma_f32_16x16x4f32 adds its four products to
-// the accumulator one after the other, each a fused multiply-add (checked bit for bit over normal,
-// subnormal and widely scaled operands), so a row's fma chain in the MFMA tile's order of inputs gives
-// the tile's sums bit for bit. That order goes in units of four inputs, the four lane groups' of one
+// the accumulator one after the other, each a fused multiply-add (the tests of the forms compare both bit for
+// bit, with ordinary weights, weights spread over 2^80, subnormal sums and overflow), so a row's fma chain in
+// the MFMA tile's order of inputs gives the tile's sums bit for bit. That order goes in units of four inputs, the four lane groups' of one
 // k-step (unit 4 q + e: the inputs kappa(L, 4 q + e, g), g < 4), and the weights are packed for it
 // (WideLayout with chain = 1): one float4 per unit and row. The inputs come from LDS, one float4 per unit
 // at the same address on every lane.
@@ -155,9 +156,8 @@ __device__ __forceinline__ void net_rows(const float4* W, const float* bias, int
 // for bit. The worlds' state is in the lanes (st, pa, rng); w: the group's world, wvalid: its lanes store.
 // Returns the lane's own action (hinge lanes; t < a.H). lds: kNetLds floats. kDuo: both waves of the world
 // call it; wave 0 forms the observation, the head and the outputs, and each takes half of a hidden layer's
-// rows, with a block barrier after the observation and after each layer (nl + 1 on either wave): one
-// wave's loads reach about 22 bytes per clock of the L2's way to its CU, two twice that. (Returns 0 on
-// wave 1.)
+// rows, with a block barrier after the observation and after each layer (nl + 1 on either wave). The two waves
+// together take 24 bytes of weights per clock (368 KB of 256-256 in 15.6k cycles). (Returns 0 on wave 1.)
 template <int kW, bool kDuo>
 __device__ __forceinline__ float wave_policy(const TileArgs& a, const LaneState& st, float pa, unsigned rng,
                                              unsigned long long seed, int N, int t, int w, int wc, bool wvalid,

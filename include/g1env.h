@@ -124,16 +124,16 @@ int g1_env_set_handover(void* h, int fences);
 /* How a physics or one-launch rollout launch of this env runs, from its batch size and hand-over mode:
  * 0 = the work queue, 1 = each world kept on two waves for the whole launch (batches that are resident
  * at once in that form: up to 1024 worlds), 2 = two worlds kept per wave (up to 4096). The same results
- * bit for bit. */
+ * bit for bit, as long as the policy's activations do not overflow. */
 int g1_env_launch_form(void* h);
 
 /* Rollout form: on = 1 (the default) runs g1_rollout as one persistent launch that interleaves the
  * policy of 16-world tiles with the physics work items, or, for batches that fit the chip at one or two
  * worlds per wave (up to 4096), keeps each wave's worlds for the whole launch (the same results bit for
- * bit); on = 0 launches the policy and the physics once per control step. The one-launch form covers every shape g1_env_set_policy accepts (two
- * hidden layers of at most 256 units on a register-resident tile, other shapes on a tile that
- * stages its activations in library-allocated device memory); g1_rollout_noalloc runs the latter
- * shapes in the per-step form. Returns 0, 1 when on = 1 but the current policy shape takes the
+ * bit); on = 0 launches the policy and the physics once per control step. The one-launch form covers
+ * every shape g1_env_set_policy accepts (two hidden layers of at most 256 units on a register-resident
+ * tile, other shapes on a tile that stages its activations in library-allocated device memory);
+ * g1_rollout_noalloc runs the latter shapes in the per-step form. Returns 0, 1 when on = 1 but the current policy shape takes the
  * per-step form, or -1 for an invalid argument. */
 int g1_env_set_fused(void* h, int on);
 
